@@ -210,9 +210,8 @@ int sd_verify_drafts(const void* logits, int32_t logits_dtype, int64_t logits_ro
  * stride >= vocab) is required and the sampled rows are decided by sd_verify_drafts's passes over it. The
  * other arguments and the outputs are sd_verify_drafts's. No counterpart in the reference for the packing (the
  * reference's F.linear reads the weight as stored). A token row's logits depend on its hidden row, the weight and
- * (vocab, hidden_dim) only, never on the call's row count (num_seqs * (K+1)) or the device's CU count: the
- * vocabulary tiles of the GEMM's last round are split along hidden_dim by a rule of (vocab, hidden_dim) alone and
- * their fp32 sums added in a fixed order in the workspace. K = 0 is plain sampling (Sampler.forward,
+ * hidden_dim only, never on the call's row count (num_seqs * (K+1)) or the device's CU count: each logit is one
+ * fp32 chain over hidden_dim in order, whichever kernel computes it. K = 0 is plain sampling (Sampler.forward,
  * sampler.py:7-16, on compute_logits' rows), so plain decode and verify steps read the same logits.
  */
 size_t sd_lm_head_packed_weight_size(int32_t vocab, int32_t hidden_dim);
@@ -232,12 +231,11 @@ int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, int32_t hid
  * computes the projections of nanovllm/layers/linear.py (the reference's qkv_proj, o_proj, gate_up_proj and
  * down_proj, nanovllm/models/qwen3.py:47-63,115-126). It is the LM head's GEMM without the argmax: packed_weight
  * is w [out_features, in_features] bf16 in sd_lm_head_pack_weight's layout (in_features a multiple of 32); x bf16
- * with 16-byte aligned rows (row stride a multiple of 8 elements), out bf16 with any row stride >= out_features. Each output row depends on its
- * input row and the weight only, never on `rows`: the library GEMM picks kernels (and summation orders) by the
- * row count, which changes a model's greedy tokens with the batch; reference counterpart of the property:
- * scripts/check_padding.py:46-52 (GEMMs, padded vs alone). The workspace size is not monotonic in `rows` (a
- * call of at most 320 rows may hold fp32 range sums that a longer call keeps in registers): size it for each
- * row count a caller uses.
+ * with 16-byte aligned rows (row stride a multiple of 8 elements), out bf16 with any row stride >= out_features.
+ * Each output row depends on its input row and the weight only, never on `rows`: the library GEMM picks kernels (and
+ * summation orders) by the row count, which changes a model's greedy tokens with the batch; reference counterpart of
+ * the property: scripts/check_padding.py:46-52 (GEMMs, padded vs alone). out may overlap x (the rows are then copied
+ * to the workspace first). The workspace size is not monotonic in `rows`: size it for each row count a caller uses.
  */
 size_t sd_linear_workspace_size(int32_t rows, int32_t out_features, int32_t in_features);
 int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, const void* packed_weight, int32_t out_features,

@@ -1,78 +1,66 @@
-// LM head over the verify rows with the verifier's argmax pass in its epilogue (replaces, for the rows the
-// verifier reads, ParallelLMHead.forward, nanovllm/layers/embed_head.py:56-68, and the first read of the
-// logits by verify_drafts, nanovllm/layers/sampler.py:66).
+// Row-invariant GEMM of the LM head and the projections: out[m, n] = bf16(sum_k x[rows[m], k] * weight[n, k]) with
+// the verifier's argmax pass in its epilogue (replaces ParallelLMHead.forward for the rows the verifier reads,
+// nanovllm/layers/embed_head.py:56-68, the first read of the logits by verify_drafts, nanovllm/layers/sampler.py:66,
+// and, without the argmax, the linear layers of nanovllm/layers/linear.py).
 //
-// logits[m, n] = bf16(sum_k hidden[rows[m], k] * weight[n, k]): the library GEMM's contract (fp32
-// accumulation, one round to bf16), with the logits_indices gather folded into the loads of hidden.
-// Shapes at Qwen3-8B: M = S (K+1) = 320 token rows, H = 4096, V = 151936 vocabulary rows: 398 GFLOP over the
-// 1.24 GB weight, about 320 FLOP per byte, at the bf16 ridge of this GPU (2.5 PF / 8 TB/s).
+// Every output element is one chain of v_mfma_f32_16x16x32_bf16 over k = 0, 32, 64, ... in fp32, rounded once to
+// bf16, whatever the kernel, its tile or the call's row count: a row's result depends on its input row and the
+// weight alone. (The reduction is never split along k. A split would put more workgroups on a short call, but its
+// fp32 sums went through memory and a second launch: 33 us of the 149 us that a 5-row call of the four Qwen3-8B
+// projections took, and 52 of 246 us at 320 rows.)
 //
-// One 8-wave workgroup owns 256 vocabulary rows and up to 320 token rows and walks H in stages of 32:
-//   * each stage's weight tile (256 x 32, 16 KB) and hidden tile (up to 320 x 32, 20 KB) are loaded straight
-//     into a ring of four LDS stages (global_load_lds_dwordx4), three stages ahead of the MFMAs: at ~12.5 B per
-//     clock per CU, the weight stream needs tens of KB in flight per CU to cover HBM latency. Both operands are
-//     packed so that a stage tile is contiguous (rows of a tile are otherwise 2 H bytes apart, and such 64-byte
-//     row pieces streamed the weight at 4.3 TB/s and the hidden rows at 6.3 TB/s from L2, measured alone). LDS
-//     rows of 64 bytes, the 16-byte chunk c of row r at slot c ^ ((r >> 2) & 3): conflict-free operand reads;
-//   * wave w takes vocabulary rows 64 (w % 4) .. +64 and token rows 32 MB (w / 4) .. +32 MB: 2 x MB
-//     v_mfma_f32_32x32x16_bf16 tiles D[n][m] = sum_k W[n][k] H[m][k] (A = weight rows, B = hidden rows, both
-//     ds_read_b128 from LDS), MB <= 5, accumulating in fp32;
-//   * epilogue: a lane holds 16 vocabulary entries of one token row per tile (the other 16 in lane l ^ 32); it
-//     rounds them to bf16, optionally stores them (the logits, for a sampling pass that reads them again), and
-//     reduces the first argmax (torch.argmax order) over the workgroup's 256 entries: its own entries in
-//     index order, the lane pair, then the four vocabulary waves through LDS. One (value, index) per token row
-//     and workgroup goes out; lm_head_merge folds them into the verifier's span statistics.
+// Packed weight (once per weight, lm_head_pack_weight): wp[t][s][r][c] = weight[256 t + r][32 s + c], rows past the
+// vocabulary zero: the 16 rows x 32 columns that one wave's A operand needs are one contiguous 1 KB block. The
+// activations are read where they are, the logits_indices gather folded into the row addresses.
+//
+//   stream_gemm  up to 16 rows: one wave per 16 or 32 weight rows, both operands straight into registers, 16 steps
+//                of 32 columns ahead. HBM bound: the weight is the traffic.
+//   tile_gemm    more rows (and few rows of a vocabulary-sized weight): a workgroup of WN x WM waves owns
+//                (16 TN WN) weight rows x (16 TM WM) token rows.
+//                  * A (weight): each wave loads its own rows into registers, DA steps of 32 columns ahead. The
+//                    weight does not pass through LDS: at 256 x 256 the LDS reads and writes of a step would take
+//                    as long as its MFMAs (128 B a clock), this way they take about 0.6 of that.
+//                  * B (tokens): stages of 64 columns (whole 128-byte lines of a row) in an LDS ring of RX slots,
+//                    loaded with global_load_lds; slot rows of 128 B, 16-byte chunk c of row r at
+//                    c ^ ((r >> 1) & 7), so that 16 rows at one chunk cover all banks. A step's operand reads are
+//                    issued one step ahead, column by column, each behind the MFMAs that used its registers.
+//                  * One barrier per two steps. The step has no branch: past the end the loads repeat the last
+//                    step's addresses (never used), so every wait is a constant count.
+//                Loads, LDS reads and MFMAs are inline asm: next to LDS DMA in flight the compiler would wait for
+//                every load before a use. Their results are tied to the waits, and every register set stays
+//                allocated until the last load has landed (tests/test_asm_gemm.py checks the compiled code).
 #pragma once
+#include <type_traits>
+
 #include "sd_common.h"
 
 namespace sd {
 namespace lmhead {
 
-constexpr int kWaves = 8;
-constexpr int kThreads = kWaves * kWave;           // 512
-constexpr int kN = 256;                            // vocabulary rows per workgroup
-constexpr int kK = 32;                             // hidden columns per stage
-constexpr int kRowBytes = kK * 2;                  // one LDS row: 64 B = 4 chunks of 16 B
-constexpr int kMaxMB = 5;                          // token blocks of 32 per wave (2 waves: 320 rows)
-constexpr int kMaxRows = 2 * kMaxMB * 32;          // 320 token rows per workgroup
-constexpr int kWBytes = kN * kRowBytes;            // 16 KB
-constexpr int kHBytes = kMaxRows * kRowBytes;      // 20 KB
-constexpr int kStageBytes = kWBytes + kHBytes;     // 36 KB
-constexpr int kRing = 4;                           // LDS stages: loads run 3 stages ahead of the MFMAs
-constexpr int kLdsBytes = kRing * kStageBytes;     // 144 KB
-constexpr int kCpolNT = 2;                         // cache policy of a load: non-temporal
+constexpr int kN = 256;                            // rows of a packed weight tile
+constexpr int kK = 32;                             // columns of a packed block: one MFMA step
+constexpr int kBlockBytes = kN * kK * 2;           // 16 KB: one step of a packed tile
+constexpr int kStreamRows = 16;                    // stream_gemm's token rows
 
-struct TileBest {  // first argmax of one token row over one workgroup's vocabulary rows
+struct TileBest {  // first argmax of one token row over one workgroup's weight rows
   float val;
   int32_t idx;
 };
 
-// Packed operands (contiguous stage tiles, so that every stage load reads whole 1 KB blocks):
-//   weight  wp[t][s][r][c] = weight[kN t + r][32 s + c]  (t < tiles, s < H / 32, r < kN, c < 32; rows past the
-//           vocabulary are 0), made once per model by lm_head_pack_weight (sd_lm_head_pack_weight);
-//   hidden  hp[s][m][c] = hidden[rows[m]][32 s + c]  (m < Mpad; rows past M are 0), made per call by
-//           lm_head_pack_hidden, which also applies the logits_indices gather.
 struct Args {
-  const uint16_t* hp;       // packed hidden [H/32][Mpad][32]
-  int32_t Mpad;             // gridDim.y * token rows per workgroup
+  const uint16_t* x;        // [*, K] bf16 rows, stride x_stride
+  int64_t x_stride;
+  const int64_t* rows;      // null (row m is token row m), or the gather; an index outside [0, x_rows) gives zeros
+  int64_t x_rows;
   int32_t M;                // token rows
-  const uint16_t* wp;       // packed weight [tiles][H/32][kN][32]
-  int32_t V, H;
-  uint16_t* logits;         // null, or [M, V] bf16 with row stride logits_stride
-  int64_t logits_stride;
-  int32_t logits_vec;       // rows 8-byte aligned: 4 entries per store
-  TileBest* best;           // [M][tiles], or null (no argmax)
-  int32_t tiles;            // vocabulary tiles of kN rows
-  // Tiles full.. (the last, partial round of workgroups) are cut into `splits` ranges of H each, one
-  // workgroup per range, so that the last round fills the GPU; such a workgroup writes its fp32 sums to
-  // `part` ([row of workgroups][tile - full][split][8 waves][2][MB][16][64 lanes]) and lm_head_fixup adds the
-  // ranges in order and runs the epilogue. splits = 1: every tile whole (full = tiles). full and splits are
-  // functions of (V, H) only and every row of workgroups uses them, so a token row's logits do not depend on
-  // how many rows the call has. The sequential form (lm_head_gemm<MB, true>) runs a split tile's ranges one
-  // after another in one workgroup and adds them in the same order in registers: the same sums, no `part`.
-  int32_t full;
-  int32_t splits;
-  float* part;
+  const uint16_t* wp;       // packed weight
+  int32_t N, K;
+  uint16_t* out;            // null, or [M, N] bf16 with row stride out_stride
+  int64_t out_stride;
+  int32_t out_vec;          // out rows 16-byte aligned: 8 entries per store
+  int32_t out_nt;           // non-temporal stores of whole lines (logits: they leave the token rows in L2)
+  TileBest* best;           // [M][tiles_n], or null (no argmax)
+  int32_t tiles_n, tiles_m;
 };
 
 // One thread per 16 bytes of the packed weight.
@@ -92,316 +80,400 @@ __global__ __launch_bounds__(256) void lm_head_pack_weight(const uint16_t* __res
   *(u32x4*)(wp + o * 8) = v;
 }
 
-// One thread per 16 bytes of the packed hidden rows (the logits_indices gather; an index outside the table
-// reads nothing and packs a zero row, and lm_head_poison marks its sequence).
-__global__ __launch_bounds__(256) void lm_head_pack_hidden(const uint16_t* __restrict__ hidden, int64_t stride,
-                                                           int32_t hidden_rows, const int64_t* __restrict__ rows,
-                                                           int32_t M, int32_t Mpad, int32_t H, uint16_t* __restrict__ hp) {
+// The call's token rows copied to dst [M][K] (gathered; an index outside the table gives a zero row), for calls
+// whose output overlaps their input. One thread per 16 bytes.
+__global__ __launch_bounds__(256) void copy_rows(const uint16_t* __restrict__ x, int64_t stride, int64_t x_rows,
+                                                 const int64_t* __restrict__ rows, int32_t M, int32_t K,
+                                                 uint16_t* __restrict__ dst) {
   const int64_t o = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int S = H / 32;
-  if (o >= (int64_t)S * Mpad * 4) return;
-  const int c8 = (int)(o % 4);
-  const int m = (int)((o / 4) % Mpad);
-  const int s = (int)(o / (4 * (int64_t)Mpad));
+  const int chunks = K / 8;
+  if (o >= (int64_t)M * chunks) return;
+  const int m = (int)(o / chunks), c = (int)(o % chunks);
+  const int64_t r = rows ? rows[m] : (int64_t)m;
   u32x4 v = {0, 0, 0, 0};
-  if (m < M) {
-    const int64_t r = rows ? rows[m] : (int64_t)m;
-    if (r >= 0 && r < hidden_rows) v = *(const u32x4*)(hidden + r * stride + 32 * s + 8 * c8);
-  }
-  *(u32x4*)(hp + o * 8) = v;
-}
-
-// LDS byte offset of 16-byte chunk c (0..3) of row r: rows of 64 B, the chunk swizzled by bits 2..3 of the row,
-// so that 16 consecutive rows at one chunk (an operand read's 16-lane pass) cover all 64 banks.
-__device__ __forceinline__ uint32_t slot(int row, int chunk) {
-  return row * kRowBytes + ((chunk ^ ((row >> 2) & 3)) << 4);
+  if (r >= 0 && r < x_rows) v = *(const u32x4*)(x + r * stride + 8 * c);
+  *(u32x4*)(dst + o * 8) = v;
 }
 
 template <int N>
 __device__ __forceinline__ void wait_vm() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N < 63 ? N : 63) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_lgkm() {
+  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N < 15 ? N : 15) : "memory");
+}
+// A value that passes through here is not read before, nor its registers reused until, this point.
+__device__ __forceinline__ void tie(bf16x8& f) { asm volatile("" : "+v"(f)); }
+
+// Accumulators in AGPRs (kAcc) where a kernel needs more than 256 registers a wave, else in VGPRs.
+template <bool kAcc>
+__device__ __forceinline__ void tie_acc(f32x4& f) {
+  if constexpr (kAcc)
+    asm volatile("" : "+a"(f));
+  else
+    asm volatile("" : "+v"(f));
+}
+template <bool kAcc>
+__device__ __forceinline__ void mfma(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  if constexpr (kAcc)
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+  else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+template <int OFF>
+__device__ __forceinline__ void lds_read(bf16x8& f, uint32_t addr) {
+  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f) : "v"(addr), "n"(OFF) : "memory");
+}
+template <bool kNT, int OFF>
+__device__ __forceinline__ void load_frag(bf16x8& f, uint32_t off, const uint8_t* base) {
+  if constexpr (kNT)
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3 nt" : "=v"(f) : "v"(off), "s"(base), "n"(OFF) : "memory");
+  else
+    asm volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(f) : "v"(off), "s"(base), "n"(OFF) : "memory");
+}
+
+// Calls f(integral_constant<I>) for I = I0 .. N - 1: registers and wait counts are indexed at compile time.
+template <int I, int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for<I + 1, N>(f);
+  }
 }
 
 typedef __attribute__((address_space(3))) void lds_void;
 
-// Epilogue, per 32-token-row block of a tile. A lane holds 16 vocabulary entries of one token row for each of
-// its two 32-row vocabulary blocks (the other 16 in lane l ^ 32): it rounds them to bf16, stores them if the
-// logits are asked for, and takes the first argmax (index order) of its entries and its lane pair's. Returns
-// it in every lane; token row m of the call (no store, the argmax still taken, for m >= M).
-__device__ __forceinline__ TileBest block_best(const Args& a, const f32x16 (&acc)[2], int n_wave, int m) {
-  const int half = (threadIdx.x % kWave) / 32;
+// The token row m (clamped to the call's rows) as a row of x; an index outside the table reads row 0 (its result
+// is replaced by zeros in the epilogue).
+__device__ __forceinline__ int64_t x_row(const Args& a, int m) {
+  m = min(m, a.M - 1);
+  if (!a.rows) return m;
+  const int64_t r = a.rows[m];
+  return r >= 0 && r < a.x_rows ? r : 0;
+}
+__device__ __forceinline__ bool row_valid(const Args& a, int m) {
+  if (!a.rows || m >= a.M) return true;
+  const int64_t r = a.rows[m];
+  return r >= 0 && r < a.x_rows;
+}
+
+// Four consecutive entries n .. n + 3 of a token row, rounded to bf16 (zeros for an invalid row) and taken into the
+// running first argmax (index order within a lane: strictly larger).
+__device__ __forceinline__ uint2 round4(const Args& a, const f32x4& acc, bool valid, int n, float& bv, int& bi) {
+  uint2 w = make_uint2(cvt_bf16x2(acc[0], acc[1]), cvt_bf16x2(acc[2], acc[3]));
+  if (!valid) w = make_uint2(0, 0);
+  if (a.best) {
+    const float v[4] = {__builtin_bit_cast(float, w.x << 16), __builtin_bit_cast(float, w.x & 0xffff0000u),
+                        __builtin_bit_cast(float, w.y << 16), __builtin_bit_cast(float, w.y & 0xffff0000u)};
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < a.N && bv == bv && !(v[e] <= bv)) {
+        bv = v[e];
+        bi = n + e;
+      }
+  }
+  return w;
+}
+// The first argmax over the four lanes that hold one token row's entries (l, l ^ 16, l ^ 32, l ^ 48).
+__device__ __forceinline__ void lanes_best(float& bv, int& bi) {
+#pragma unroll
+  for (int off = 16; off <= 32; off <<= 1) {
+    const float ov = __shfl_xor(bv, off);
+    const int oi = __shfl_xor(bi, off);
+    if (better(ov, oi, bv, bi)) {
+      bv = ov;
+      bi = oi;
+    }
+  }
+}
+
+// Up to 16 token rows. Lane l holds row l % 16 of both operands, columns 8 (l / 16) .. + 7 of each step; one wave takes
+// 16 TN weight rows, kStreamDepth steps of 32 columns ahead. More rows a wave read the token rows fewer times per byte
+// of weight, fewer keep a small matrix spread over the GPU (row_plan): at 5 rows 4096 x 12288 took 21.0 / 24.3 us
+// with 16 / 32 rows a wave, 24576 x 4096 44.2 / 35.9 us (5.6 TB/s).
+constexpr int kStreamDepth = 16;
+template <int TN>
+__global__ __launch_bounds__(kWave) void stream_gemm(Args a) {
+  constexpr int D = kStreamDepth;
+  const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
+  const int S = a.K / kK;
+  const int n0 = blockIdx.x * 16 * TN;
+  const uint8_t* wsrc =
+      (const uint8_t*)a.wp + (int64_t)(n0 / kN) * S * kBlockBytes + (n0 % kN) * 64 + r16 * 64 + g * 16;
+  const uint8_t* xsrc = (const uint8_t*)(a.x + x_row(a, r16) * a.x_stride) + g * 16;
+  bf16x8 fa[D][TN], fb[D];
+  f32x4 acc[TN];
+#pragma unroll
+  for (int i = 0; i < TN; ++i) acc[i] = f32x4{};
+  auto load = [&](int t, bf16x8 (&fa)[TN], bf16x8& fb) {   // past the end: the last step again, never used
+    const int s = min(t, S - 1);
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      fa[i] = __builtin_nontemporal_load((const bf16x8*)(wsrc + (int64_t)s * kBlockBytes + i * 1024));
+    fb = *(const bf16x8*)(xsrc + (int64_t)s * 64);
+  };
+  auto step = [&](int d) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[d][i], fb[d], acc[i], 0, 0, 0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, fa[d], fb[d]);
+  int t = 0;
+  for (; t + D <= S; t += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      step(d);
+      load(t + d + D, fa[d], fb[d]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (t + d < S) step(d);
+  const bool valid = row_valid(a, r16);
   float bv = -INFINITY;
   int bi = 0x7fffffff;
 #pragma unroll
-  for (int nb = 0; nb < 2; ++nb) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int nf = n_wave + 32 * nb + 8 * g + 4 * half;  // first of 4 consecutive entries
-      float v[4];
-      uint16_t bits[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        bits[e] = f32_to_bf16_bits(acc[nb][4 * g + e]);
-        v[e] = bf16_bits_to_f32(bits[e]);
-      }
-      if (a.logits && m < a.M) {
-        uint16_t* dst = a.logits + (int64_t)m * a.logits_stride + nf;
-        if (nf + 3 < a.V && a.logits_vec) {
-          *(uint2*)dst = make_uint2((uint32_t)bits[0] | ((uint32_t)bits[1] << 16),
-                                    (uint32_t)bits[2] | ((uint32_t)bits[3] << 16));
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (nf + e < a.V) dst[e] = bits[e];
-        }
-      }
+  for (int i = 0; i < TN; ++i) {
+    const int n = n0 + 16 * i + 4 * g;
+    const uint2 w = round4(a, acc[i], valid, n, bv, bi);
+    if (!a.out || r16 >= a.M) continue;
+    uint16_t* dst = a.out + (int64_t)r16 * a.out_stride + n;
+    if (n + 3 < a.N && a.out_vec) {
+      *(uint2*)dst = w;
+    } else {
+      const uint16_t bits[4] = {(uint16_t)w.x, (uint16_t)(w.x >> 16), (uint16_t)w.y, (uint16_t)(w.y >> 16)};
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (nf + e < a.V && bv == bv && !(v[e] <= bv)) {  // index order within the lane: strictly larger
-          bv = v[e];
-          bi = nf + e;
-        }
+        if (n + e < a.N) dst[e] = bits[e];
     }
   }
-  const float ov = __shfl_xor(bv, 32);
-  const int oi = __shfl_xor(bi, 32);
-  if (better(ov, oi, bv, bi)) {
-    bv = ov;
-    bi = oi;
+  if (a.best) {
+    lanes_best(bv, bi);
+    if (g == 0 && r16 < a.M) a.best[(int64_t)r16 * a.tiles_n + blockIdx.x] = TileBest{bv, bi};
   }
-  return TileBest{bv, bi};
 }
 
-// The four vocabulary waves' candidates of `rows` token rows (red[row][wave], in LDS, after a barrier), reduced
-// in wave order into best[m][tile] by threads 0.. of the workgroup.
-__device__ __forceinline__ void reduce_best(const Args& a, const TileBest* red, int rows, int m0, int tile) {
-  if (!a.best) return;  // a plain linear layer: the logits only
-  for (int mr = threadIdx.x; mr < rows; mr += blockDim.x) {
-    const int m = m0 + mr;
-    if (m >= a.M) continue;
-    TileBest b = red[mr * 4];
+// One workgroup shape of tile_gemm. DA: register sets of weight (steps ahead + 1, even); RX: LDS slots of token
+// stages; kAcc: accumulators in AGPRs; kNT: the weight non-temporal (shapes that mostly read it once).
+template <int TN_, int TM_, int WN_, int WM_, int DA_, int RX_, bool kAcc_, bool kNT_>
+struct Tile {
+  static constexpr int TN = TN_, TM = TM_, WN = WN_, WM = WM_, DA = DA_, RX = RX_;
+  static constexpr bool kAcc = kAcc_, kNT = kNT_;
+  static constexpr int kWaves = WN * WM, kThreads = kWaves * kWave;
+  static constexpr int kRowsN = 16 * TN * WN, kRowsM = 16 * TM * WM;
+  static constexpr int kSlot = kRowsM * 128;                         // one stage of 64 columns
+  static constexpr int kPieces = (kRowsM / 8 + kWaves - 1) / kWaves;  // 1 KB loads of a stage per wave
+  static_assert(DA % 2 == 0 && 2 * (RX - 2) >= DA - 2, "the stages ahead cover the steps ahead");
+  static_assert(kN % kRowsN == 0 && TN <= 4, "a workgroup's weight rows lie in one packed tile");
+  static_assert(TM <= 16, "lgkmcnt counts the reads ahead");
+  static constexpr int kRing = RX * kSlot, kRed = kRowsM * WN * (int)sizeof(TileBest);
+  static_assert(kRing + kRed <= 160 * 1024 && kRowsM * kRowsN * 2 <= kRing, "the ring takes the output tile");
+};
+
+template <class T>
+__global__ __launch_bounds__(T::kThreads, 1) void tile_gemm(Args a) {
+  constexpr int TN = T::TN, TM = T::TM, WN = T::WN, DA = T::DA, RX = T::RX, PX = T::kPieces;
+  constexpr int XS = T::kSlot, MT = T::kRowsM;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[T::kRing + T::kRed];
+  const int lane = threadIdx.x % kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int wn = wave % WN, wm = wave / WN;
+  const int S = a.K / kK, nst = (S + 1) / 2;
+  // Workgroups go round-robin over the 8 XCDs: XCD k takes the weight tiles k, k + 8, ..., all token tiles of one
+  // before the next, so that a weight tile is read from HBM by one XCD's L2 only.
+  const int xcd = blockIdx.x % 8, j0 = blockIdx.x / 8;
+  const int nt = xcd + 8 * (j0 / a.tiles_m), mt = j0 % a.tiles_m;
+  if (nt >= a.tiles_n) return;
+  const int m0 = mt * MT;
+  const int nw = nt * T::kRowsN + wn * TN * 16;   // this wave's first weight row
+  const uint8_t* wbase = (const uint8_t*)a.wp + (int64_t)(nw / kN) * S * kBlockBytes + (nw % kN) * 64;
+  const uint32_t wlane = (lane % 16) * 64 + (lane / 16) * 16;
+
+  // Token loads: lane l's 16 bytes land at the instruction's LDS base + 16 l: row l / 8 of the piece's 8 rows,
+  // physical chunk l % 8, so the lane fetches the logical chunk that the swizzle puts there.
+  uint64_t xsrc[PX];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
-      const TileBest o = red[mr * 4 + w];
+  for (int i = 0; i < PX; ++i) {
+    const int r = 8 * min(wave * PX + i, MT / 8 - 1) + lane / 8;
+    xsrc[i] = (uint64_t)(a.x + x_row(a, m0 + r) * a.x_stride + 8 * ((lane % 8) ^ ((r >> 1) & 7)));
+    asm volatile("" : "+v"(xsrc[i]));
+  }
+  const int half_stage = S % 2 ? nst - 1 : -1;  // a last stage of 32 columns: its upper chunks repeat the lower ones
+  auto load_x = [&](int st, uint32_t slot, int i) __attribute__((always_inline)) {
+    const int q = min(wave * PX + i, MT / 8 - 1);
+    uint64_t p = xsrc[i] + (uint64_t)(uint32_t)(st * 128);
+    if (st == half_stage && ((lane % 8) ^ (((8 * q + lane / 8) >> 1) & 7)) >= 4) p -= 64;
+    __builtin_amdgcn_global_load_lds((const void*)p, (lds_void*)(lds + slot + q * 1024), 16, 0, 0);
+  };
+
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      acc[i][j] = f32x4{};
+      tie_acc<T::kAcc>(acc[i][j]);
+    }
+  asm volatile("s_nop 7");
+  const int r16 = lane % 16, g = lane / 16;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
+  const uint32_t swz = (r16 >> 1) & 7;
+  const uint32_t brow = lds0 + (wm * TM * 16 + r16) * 128;
+  const uint32_t boff[2] = {brow + ((g ^ swz) << 4), brow + (((4 + g) ^ swz) << 4)};  // even / odd step of a stage
+
+  bf16x8 fa[DA][TN], fb[TM];
+  uint32_t xw = (RX - 1) * XS, xr = 0;   // slots of the next stage to load and of the stage being read
+  // Step t: the MFMAs of columns 32 t .. + 31. Behind each token block's MFMAs its next operand read goes out, and
+  // the step's loads (the weight of step t + DA - 1; in odd steps the token stage RX - 1 ahead) are spread over
+  // the blocks. kLoad = false: the last steps of a K that is not a multiple of 32 DA, everything already loaded.
+  auto step = [&](int t, auto dc, auto loadc) __attribute__((always_inline)) {
+    constexpr int d = decltype(dc)::value, prev = (d + DA - 1) % DA, odd = d % 2;
+    constexpr bool kLoad = decltype(loadc)::value;
+    // Loads issued after those this step needs: its own weight (issued at the end of step t - DA + 1) and, in an
+    // odd step, the next stage's tokens (issued in step t - 2 (RX - 2)).
+    constexpr int kAfterA = (DA - 2) * TN + (DA / 2 - 1) * PX, kAfterX = 2 * (RX - 2) * TN + (RX - 3) * PX;
+    if constexpr (kLoad) wait_vm<odd && kAfterX < kAfterA ? kAfterX : kAfterA>();
+    static_for<0, TN>([&](auto i) { tie(fa[d][decltype(i)::value]); });
+    if constexpr (odd) {
+      // every wave's part of the next stage has landed, and every wave is done with the stage before this one
+      if constexpr (kLoad) __builtin_amdgcn_s_barrier();
+      xr = xr + XS == RX * XS ? 0 : xr + XS;
+    }
+    const int xst = min((t - 1) / 2 - 1 + RX, nst - 1);
+    const uint32_t baddr = boff[1 - odd] + xr;
+    const uint8_t* wnext = wbase + (uint64_t)(uint32_t)min(t + DA - 1, S - 1) * kBlockBytes;
+    constexpr int kX = odd ? PX : 0, kItems = kX + TN;
+    static_for<0, TM>([&](auto jc) {
+      constexpr int j = decltype(jc)::value;
+      wait_lgkm<TM - 1>();
+      tie(fb[j]);
+      static_for<0, TN>([&](auto i) {
+        mfma<T::kAcc>(acc[decltype(i)::value][j], fa[d][decltype(i)::value], fb[j]);
+      });
+      lds_read<j * 2048>(fb[j], baddr);
+      if constexpr (kLoad)
+        static_for<j * kItems / TM, (j + 1) * kItems / TM>([&](auto kc) {
+          constexpr int k = decltype(kc)::value;
+          if constexpr (k < kX)
+            load_x(xst, xw, k);
+          else
+            load_frag<T::kNT, (k - kX) * 1024>(fa[prev][k - kX], wlane, wnext);
+        });
+    });
+    if constexpr (odd) xw = xw + XS == RX * XS ? 0 : xw + XS;
+  };
+
+  for (int st = 0; st < RX - 1; ++st)
+#pragma unroll
+    for (int i = 0; i < PX; ++i) load_x(min(st, nst - 1), st * XS, i);
+  static_for<0, DA - 1>([&](auto d) {
+    const uint8_t* p = wbase + (uint64_t)(uint32_t)min((int)decltype(d)::value, S - 1) * kBlockBytes;
+    static_for<0, TN>([&](auto i) {
+      load_frag<T::kNT, decltype(i)::value * 1024>(fa[decltype(d)::value][decltype(i)::value], wlane, p);
+    });
+  });
+  wait_vm<0>();
+  __builtin_amdgcn_s_barrier();
+  static_for<0, TM>([&](auto j) { lds_read<decltype(j)::value * 2048>(fb[decltype(j)::value], boff[0]); });
+  int t = 0;
+  for (; t + DA <= S; t += DA)
+    static_for<0, DA>([&](auto d) { step(t + decltype(d)::value, d, std::true_type{}); });
+  // Nothing in flight past here; until here no register set was free for another value.
+  wait_vm<0>();
+  static_for<0, DA - 1>([&](auto d) {
+    static_for<0, TN>([&](auto i) { tie(fa[decltype(d)::value][decltype(i)::value]); });
+  });
+  if (t < S) {
+    __builtin_amdgcn_s_barrier();
+    static_for<0, DA - 1>([&](auto d) {
+      if (t + decltype(d)::value < S) step(t + decltype(d)::value, d, std::false_type{});
+    });
+  }
+  wait_lgkm<0>();
+  static_for<0, TM>([&](auto j) { tie(fb[decltype(j)::value]); });
+  asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMAs' results before the VALU reads them
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) tie_acc<T::kAcc>(acc[i][j]);
+
+  // ---- epilogue: a lane holds entries 16 i + 4 g .. + 3 of token row 16 j + r16. The rounded tile goes through the
+  // ring's bytes (row mr of 2 NT bytes, 16-byte chunk c at c ^ (mr % 16)), so that the stores cover whole lines: with
+  // 8-byte stores from the accumulators the LM head at 320 rows took 20 us longer with its logits than without ----
+  constexpr int NT = T::kRowsN, kChunks = NT / 8, kSwz = (kChunks < 16 ? kChunks : 16) - 1;
+  TileBest* red = (TileBest*)(lds + T::kRing);  // [MT][WN]
+  __syncthreads();                              // every wave's last reads of the ring
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int mr = wm * TM * 16 + 16 * j + r16;
+    const bool valid = row_valid(a, m0 + mr);
+    float bv = -INFINITY;
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int nr = wn * TN * 16 + 16 * i + 4 * g;
+      const uint2 w = round4(a, acc[i][j], valid, nt * NT + nr, bv, bi);
+      *(uint2*)(lds + mr * (2 * NT) + (((nr / 8) ^ (mr & kSwz)) << 4) + 8 * (g % 2)) = w;
+    }
+    if (a.best) {
+      lanes_best(bv, bi);
+      if (g == 0) red[mr * WN + wn] = TileBest{bv, bi};
+    }
+  }
+  __syncthreads();
+  const int rows = min(MT, a.M - m0), cols = min(NT, a.N - nt * NT);
+  if (a.out) {
+    uint16_t* out = a.out + (int64_t)m0 * a.out_stride + nt * NT;
+    if (a.out_vec && cols == NT) {
+      auto store_rows = [&](auto ntc) __attribute__((always_inline)) {
+        for (int idx = threadIdx.x; idx < rows * kChunks; idx += T::kThreads) {
+          const int mr = idx / kChunks, c = idx % kChunks;
+          const u32x4 w = *(const u32x4*)(lds + mr * (2 * NT) + ((c ^ (mr & kSwz)) << 4));
+          u32x4* dst = (u32x4*)(out + mr * a.out_stride + 8 * c);
+          if constexpr (decltype(ntc)::value)
+            __builtin_nontemporal_store(w, dst);
+          else
+            *dst = w;
+        }
+      };
+      if (a.out_nt)
+        store_rows(std::true_type{});
+      else
+        store_rows(std::false_type{});
+    } else {
+      for (int idx = threadIdx.x; idx < rows * NT; idx += T::kThreads) {
+        const int mr = idx / NT, n = idx % NT;
+        if (n < cols)
+          out[mr * a.out_stride + n] =
+              *(const uint16_t*)(lds + mr * (2 * NT) + (((n / 8) ^ (mr & kSwz)) << 4) + 2 * (n % 8));
+      }
+    }
+  }
+  if (!a.best) return;
+  for (int mr = threadIdx.x; mr < rows; mr += T::kThreads) {
+    TileBest b = red[mr * WN];
+#pragma unroll
+    for (int w = 1; w < WN; ++w) {
+      const TileBest o = red[mr * WN + w];
       if (better(o.val, o.idx, b.val, b.idx)) b = o;
     }
-    a.best[(int64_t)m * a.tiles + tile] = b;
+    a.best[(int64_t)(m0 + mr) * a.tiles_n + nt] = b;
   }
 }
 
-template <int MB, bool kSeq = false>
-__global__ __launch_bounds__(kThreads) void lm_head_gemm(Args a) {
-  static_assert(MB >= 1 && MB <= kMaxMB, "token blocks per wave");
-  static_assert(!kSeq || MB <= 2, "the sequential ranges keep a second accumulator set");
-  constexpr int kRows = 2 * MB * 32;               // token rows of this workgroup
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kLdsBytes];
-  const int tid = threadIdx.x;
-  const int lane = tid % kWave;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-  const int wn = wave % 4, wm = wave / 4;
-  // This workgroup's tile and range of H stages (the whole of H, or one range of a split tile).
-  const int S = a.H / kK;
-  int tile = blockIdx.x, split = -1, s_begin = 0, nstages = S;
-  if (!kSeq && (int)blockIdx.x >= a.full) {
-    const int j = blockIdx.x - a.full;
-    tile = a.full + j / a.splits;
-    split = j % a.splits;
-    s_begin = split * S / a.splits;
-    nstages = (split + 1) * S / a.splits - s_begin;
-  }
-  const int m0 = blockIdx.y * kRows;
-
-  // Stage loads straight into LDS (global_load_lds_dwordx4: lane l's 16 bytes land at the instruction's LDS
-  // base + 16 l, i.e. row l / 4, physical chunk l % 4 of a 16-row group; so the lane fetches the logical chunk
-  // that the swizzle puts there: each instruction reads one contiguous 1 KB block of a packed operand). Waves
-  // 0-3 load the weight tile (4 groups of 16 rows each), waves 4-7 the hidden tile (MB groups each).
-  const int lrow = lane / 4, lchunk = (lane % 4) ^ ((lane / 16) & 3);
-  const uint32_t lane_off = lrow * 32 + 8 * lchunk;   // elements within a 16-row group
-  const bool wloader = wave < 4;
-  constexpr int kLoads = MB > 4 ? MB : 4;          // instructions per stage of the busiest loader
-  const int nloads = wloader ? 4 : MB;
-  uint32_t loff[kLoads], goff[kLoads];             // LDS offset; element offset within the stage tile
-#pragma unroll
-  for (int i = 0; i < kLoads; ++i) {
-    const int g = wloader ? 4 * wave + i : MB * (wave - 4) + min(i, MB - 1);
-    goff[i] = 16 * g * 32 + lane_off;
-    loff[i] = (wloader ? 0 : kWBytes) + 16 * g * kRowBytes;
-  }
-  // Every workgroup walks its stages in order from s_begin, so the workgroups of a round read the same hidden
-  // stage at about the same time, and the weight, read once, streams with the non-temporal policy: both keep
-  // the hidden rows in L2 (FETCH_SIZE 2.39 -> 1.28 GB per call against rotated starts and default loads, and
-  // 455 -> 443 us).
-  auto issue = [&](int st) {
-    uint8_t* ring = lds + (st % kRing) * kStageBytes;
-    const int ks = s_begin + st;
-    const uint16_t* base = wloader ? a.wp + ((int64_t)tile * S + ks) * (kN * kK)
-                                   : a.hp + ((int64_t)ks * a.Mpad + m0) * kK;
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-      if (i < nloads) {
-        if (wloader)
-          __builtin_amdgcn_global_load_lds((const void*)(base + goff[i]), (lds_void*)(ring + loff[i]), 16, 0, kCpolNT);
-        else
-          __builtin_amdgcn_global_load_lds((const void*)(base + goff[i]), (lds_void*)(ring + loff[i]), 16, 0, 0);
-      }
-  };
-  // Waits until this wave's loads of a stage have landed, given how many later stages it has issued.
-  auto wait_stage = [&](int later) {
-    if (wloader) {
-      if (later >= 3) wait_vm<12>(); else if (later == 2) wait_vm<8>(); else if (later == 1) wait_vm<4>(); else wait_vm<0>();
-    } else {
-      if (later >= 3) wait_vm<3 * MB>(); else if (later == 2) wait_vm<2 * MB>(); else if (later == 1) wait_vm<MB>();
-      else wait_vm<0>();
-    }
-  };
-
-  f32x16 acc[2][MB];
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = f32x16{};
-
-  const int col = lane % 32, half = lane / 32;
-  // Operand fragments of one 16-deep step (ks 0 or 1) of ring slot `buf`.
-  auto read_frags = [&](int buf, int ks, bf16x8 (&af)[2], bf16x8 (&bfr)[MB]) {
-    const uint8_t* wbuf = lds + buf * kStageBytes;
-    const uint8_t* hbuf = wbuf + kWBytes;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb) af[nb] = *(const bf16x8*)(wbuf + slot(64 * wn + 32 * nb + col, 2 * ks + half));
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb) bfr[mb] = *(const bf16x8*)(hbuf + slot(MB * 32 * wm + 32 * mb + col, 2 * ks + half));
-  };
-  auto mfmas = [&](const bf16x8 (&af)[2], const bf16x8 (&bfr)[MB]) {
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-        acc[nb][mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[nb], bfr[mb], acc[nb][mb], 0, 0, 0);
-  };
-  // The hand-off between stages sits in the middle of a stage: once this wave's second-step fragments of
-  // stage s are in registers, it waits for stage s+1's loads and the barrier (after which every wave is done
-  // reading stage s, so its slot takes stage s+4), reads stage s+1's first-step fragments, and only then
-  // runs stage s's second-step MFMAs: operand reads overlap MFMAs on both sides of the barrier.
-  auto handoff = [&](int next) {  // `next` = the stage about to be read
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    wait_stage(min(nstages - 1 - next, 2));
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (next + 3 < nstages) issue(next + 3);
-  };
-  // The sequential form: a split tile's range r covers stages r S / splits .. (r + 1) S / splits - 1 (the
-  // physical split's ranges); each is summed from zero, and the ranges are added in order into `sum`, as
-  // lm_head_fixup adds them.
-  const int nranges = kSeq && tile >= a.full ? a.splits : 1;
-  int range = 0, range_end = S / nranges;
-  f32x16 sum[2][kSeq ? MB : 1];
-  auto fold = [&]() {
-    if constexpr (kSeq) {
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-          sum[nb][mb] = range == 0 ? acc[nb][mb] : sum[nb][mb] + acc[nb][mb];
-          acc[nb][mb] = f32x16{};
-        }
-    }
-  };
-  bf16x8 a0[2], b0[MB], a1[2], b1[MB];
-  for (int st = 0; st < 3 && st < nstages; ++st) issue(st);
-  handoff(0);
-  read_frags(0, 0, a0, b0);
-  // The last stage is peeled: a loop body without a branch between the hand-off's operand reads and the
-  // second-step MFMAs lets those MFMAs wait only for their own (older) reads, not for the next stage's.
-  for (int s = 0; s + 1 < nstages; ++s) {
-    read_frags(s % kRing, 1, a1, b1);
-    mfmas(a0, b0);
-    handoff(s + 1);
-    read_frags((s + 1) % kRing, 0, a0, b0);
-    mfmas(a1, b1);
-    if constexpr (kSeq) {
-      if (s + 1 == range_end) {  // stage s ends range `range` (registers only: no memory operation)
-        fold();
-        ++range;
-        range_end = (range + 1) * S / nranges;
-      }
-    }
-  }
-  read_frags((nstages - 1) % kRing, 1, a1, b1);
-  mfmas(a0, b0);
-  mfmas(a1, b1);
-  if constexpr (kSeq) {
-    if (nranges > 1) {  // the last range, added last
-#pragma unroll
-      for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) acc[nb][mb] = sum[nb][mb] + acc[nb][mb];
-    }
-  }
-
-  if (split >= 0) {
-    // ---- one range of a split tile: the fp32 sums out, lm_head_fixup finishes the tile ----
-    const int64_t range = (int64_t)blockIdx.y * (a.tiles - a.full) * a.splits + (blockIdx.x - a.full);
-    float* dst = a.part + (range * kWaves + wave) * (2 * MB * 16 * kWave) + lane;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) dst[((nb * MB + mb) * 16 + r) * kWave] = acc[nb][mb][r];
-    return;
-  }
-  // ---- epilogue: per token row, the first argmax over the workgroup's 256 vocabulary rows ----
-  __syncthreads();  // every wave's last stage read: the ring is free for the reduction
-  TileBest* red = (TileBest*)lds;  // [kRows][4]
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-    const int mr = MB * 32 * wm + 32 * mb + col;  // token row within the workgroup
-    const f32x16 blk[2] = {acc[0][mb], acc[1][mb]};
-    const TileBest b = block_best(a, blk, tile * kN + 64 * wn, m0 + mr);
-    if (half == 0) red[mr * 4 + wn] = b;
-  }
-  __syncthreads();
-  reduce_best(a, red, kRows, m0, tile);
-}
-
-// The tiles split along H: one 4-wave workgroup per (split tile, 32-token-row block, row of GEMM workgroups)
-// adds the ranges' sums in range order and finishes the block as lm_head_gemm's epilogue does. Wave w takes
-// the vocabulary rows of the GEMM's wave w of the block's token half: 64 w .. 64 w + 63.
-template <int MB>
-__global__ __launch_bounds__(256) void lm_head_fixup(Args a) {
-  __shared__ TileBest red[32 * 4];
-  const int lane = threadIdx.x % kWave;
-  const int wn = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int wm = blockIdx.y / MB, mb = blockIdx.y % MB;
-  const int tile = a.full + blockIdx.x;
-  const int m0 = blockIdx.z * (2 * MB * 32);       // first token row of the GEMM's row of workgroups
-  constexpr int kPerWave = 2 * MB * 16 * kWave;
-  const int64_t range0 = ((int64_t)blockIdx.z * (a.tiles - a.full) + blockIdx.x) * a.splits;
-  const float* src = a.part + (range0 * kWaves + 4 * wm + wn) * kPerWave + mb * 16 * kWave + lane;
-  f32x16 acc[2];
-#pragma unroll
-  for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[nb][r] = src[(nb * MB * 16 + r) * kWave];
-  for (int sp = 1; sp < a.splits; ++sp) {
-    const float* p = src + (int64_t)sp * kWaves * kPerWave;
-    float t[2][16];
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) t[nb][r] = p[(nb * MB * 16 + r) * kWave];
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[nb][r] += t[nb][r];
-  }
-  const int col = lane % 32;
-  const int mr = MB * 32 * wm + 32 * mb + col;
-  const TileBest b = block_best(a, acc, tile * kN + 64 * wn, m0 + mr);
-  if (lane < 32) red[col * 4 + wn] = b;
-  __syncthreads();
-  reduce_best(a, red, 32, m0 + MB * 32 * wm + 32 * mb, tile);
-}
+// The workgroup shapes, smallest first: the larger, the less is loaded per MFMA (row_plan chooses).
+typedef Tile<1, 4, 2, 1, 16, 9, true, true> Tile32x64;
+typedef Tile<1, 5, 2, 1, 16, 9, true, true> Tile32x80;
+typedef Tile<1, 5, 4, 1, 8, 6, true, true> Tile64x80;
+typedef Tile<2, 4, 4, 1, 8, 6, true, true> Tile128x64;
+typedef Tile<2, 5, 4, 1, 8, 6, true, true> Tile128x80;
+typedef Tile<2, 10, 4, 1, 8, 6, true, false> Tile128x160;
+typedef Tile<4, 2, 4, 1, 8, 6, false, true> Tile256x32;
+typedef Tile<4, 8, 4, 1, 8, 6, true, false> Tile256x128;
+typedef Tile<4, 10, 4, 1, 8, 6, true, true> Tile256x160;
+typedef Tile<4, 16, 4, 1, 4, 4, true, false> Tile256x256;
 
 }  // namespace lmhead
 }  // namespace sd

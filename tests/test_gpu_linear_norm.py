@@ -112,3 +112,35 @@ def test_rms_norm_rows_independent_of_row_count_and_in_place(device):
     want_out, want_res = norm(x[:64], r[:64])
     rms_norm(xi, norm.weight.data, norm.eps, ri, out=xi, residual_out=ri)
     assert torch.equal(xi, want_out) and torch.equal(ri, want_res)
+
+
+# Edges of the row-invariant GEMM's kernels: the 16-row stream, each workgroup shape one row short of, at and past its
+# rows, columns that are no multiple of the two-step stages or of the steps ahead (32, 96, 160, 544), weight rows that
+# end inside a tile and inside a store of four, an unaligned output stride. Every row equals its own one-row call
+# (bitwise) and the float64 product within the bound above.
+@pytest.mark.parametrize("N,K", [(1000, 32), (515, 96), (2053, 160), (4096, 544), (6150, 256), (24576, 64)])
+def test_linear_kernel_edges(device, N, K):
+    g = torch.Generator(device=device).manual_seed(N + K)
+    x = torch.randn(1100, K, device=device, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, device=device, generator=g) * K ** -0.5).to(torch.bfloat16)
+    lin = RowInvariantLinear(w)
+    probes = [0, 1, 15, 16, 63, 79, 127, 159, 160, 255, 256, 1099]
+    alone = torch.cat([lin(x[r:r + 1]) for r in probes])
+    _check_rows(x, w, lin(x[:17]), [0, 15, 16])
+    for M in (15, 16, 17, 64, 65, 80, 81, 128, 160, 161, 256, 257, 640, 1100):
+        wide = torch.full((M, N + 3), 7.0, dtype=torch.bfloat16, device=device)   # rows not 8-byte aligned
+        print(f"M={M} N={N} K={K}", flush=True)
+        y = lin(x[:M], out=wide[:, 1:1 + N])
+        assert bool((wide[:, 0] == 7).all()) and bool((wide[:, 1 + N:] == 7).all())
+        for i, r in enumerate(probes):
+            if r < M:
+                assert torch.equal(y[r], alone[i]), f"row {r} of {M}"
+
+
+def test_linear_output_over_its_input(device):
+    g = torch.Generator(device=device).manual_seed(5)
+    lin = RowInvariantLinear((torch.randn(512, 512, device=device, generator=g) / 23).to(torch.bfloat16))
+    for M in (3, 100, 700):
+        x = torch.randn(M, 512, device=device, generator=g).to(torch.bfloat16)
+        want = lin(x)
+        assert torch.equal(lin(x, out=x), want)
