@@ -94,7 +94,7 @@ int sd_qk_norm_rope_store(const void* q, int64_t q_row_stride, const void* k, in
  * num_query_tokens or the other rows (bitwise), and equals the row's result from sd_varlen_attention.
  * sd_paged_decode needs the workspace only when the call has too few (sequence, KV head) pairs to merge
  * inside one workgroup (residue partials); sd_paged_decode_workspace_size also counts the sequence order
- * of the planned variant below.
+ * and arrival counts of the planned variant below.
  */
 size_t sd_paged_decode_workspace_size(int32_t num_seqs, int32_t num_query_tokens, int32_t num_heads,
                                       int32_t num_kv_heads, int32_t head_dim, int32_t block_size,
@@ -116,8 +116,10 @@ int sd_paged_decode(const void* q, int64_t q_token_stride, const void* k_cache, 
  * the mean), the default policy otherwise; sd_paged_decode always loads non-temporal. Order and policy only
  * decide which workgroup computes which sequence and how it loads: results are bitwise those of
  * sd_paged_decode even when the plan was made for other context lengths, as long as it was made for the
- * same num_seqs. No counterpart
- * in the reference; it serves the per-layer loop of a decode step (nanovllm/engine/model_runner.py:476-485).
+ * same num_seqs. With too few pairs to merge inside one workgroup, the planned call's last workgroup of a pair
+ * merges its partials (the plan clears the arrival counts in the workspace, each call leaves them cleared).
+ * No counterpart in the reference; it serves the per-layer loop of a decode step
+ * (nanovllm/engine/model_runner.py:476-485).
  */
 int sd_paged_decode_plan(const int32_t* context_lens, int32_t num_seqs, int32_t num_query_tokens, int32_t num_heads,
                          int32_t num_kv_heads, void* workspace, size_t workspace_bytes, void* stream);

@@ -111,6 +111,7 @@ struct Params {
   int64_t out_stride;
   float* part_o;                // [item][Hkv][kResidues][rows_alloc][kD]
   float* part_ml;               // [item][Hkv][kResidues][rows_alloc][2] = (max, sum)
+  int32_t* arrivals;            // [item][Hkv] workgroups of the pair that are done, or null: attn_combine merges
   int32_t wave_slots;           // workgroups the GPU runs at once (one per CU): the head rotation period
 };
 
@@ -194,6 +195,87 @@ __device__ __forceinline__ T kv_load(const uint8_t* ptr) {
 // out = O / L (0 when L == 0). Explicit fmas keep the rounding identical in both places.
 __device__ __forceinline__ float merge_scale(float m_r, float M) {
   return exp2_fast(m_r - (M == -INFINITY ? 0.f : M));
+}
+
+// A residue's partials. kThrough: decode calls that merge_last may finish, whose workgroups run on several XCDs with
+// an L2 each: stores at agent scope (written through) and loads at agent scope, so that no fence has to write back or
+// drop an L2. With release and acquire fences instead, B=1 took 14.3 us a layer, against 12.7 with attn_combine.
+constexpr int kCpolAgent = 16;  // sc1
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t partials_rsrc(const Params& p) {
+  return __builtin_amdgcn_make_buffer_rsrc(p.part_o, 0, 0x7fffffff, 0x00020000);
+}
+template <bool kThrough>
+__device__ __forceinline__ void store_partial(const Params& p, int64_t cell, int d, f32x4 o) {
+  if constexpr (kThrough)
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), partials_rsrc(p),
+                                           (uint32_t)((cell * kD + d) * sizeof(float)), 0, kCpolAgent);
+  else
+    *(f32x4*)(p.part_o + cell * kD + d) = o;
+}
+template <bool kThrough>
+__device__ __forceinline__ void store_max_sum(const Params& p, int64_t cell, float m, float l) {
+  const float2 v = {m, l};
+  if constexpr (kThrough)
+    __hip_atomic_store((uint64_t*)(p.part_ml + cell * 2), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  else
+    *(float2*)(p.part_ml + cell * 2) = v;
+}
+
+// Called by every thread of a workgroup whose partials of the pair (item, h) are written: the last of the pair's
+// `wgs` workgroups to come here merges the eight partials and writes the pair's rows; `lds` is free. Every wave waits
+// for its stores before the workgroup arrives. The arrival count is 0 between launches: the plan clears it and the
+// last workgroup resets it. The merge as a kernel of its own took 3.9-4.8 us and its launch; here it is one round trip
+// for the arrival and one for the partials (8 layers of B=1, 1500 keys: 102 -> 94-96 us; 4 layers of B=16, k=4: 199 ->
+// 197). Each thread finishes four consecutive d of one row, with attn_combine's fma chain.
+__device__ __forceinline__ void merge_last(const Params& p, uint8_t* lds, const Item& it, int item, int h, int wgs,
+                                           int threads) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are stored
+  __syncthreads();
+  const int64_t pair = (int64_t)item * p.Hkv + h;
+  int32_t* flag = (int32_t*)lds;
+  if (threadIdx.x == 0) {
+    const int before = __hip_atomic_fetch_add(p.arrivals + pair, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool last = before == wgs - 1;
+    if (last) __hip_atomic_store(p.arrivals + pair, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    *flag = last;
+  }
+  __syncthreads();
+  if (*flag == 0) return;
+  const int rows = it.np * p.g;
+  const __amdgpu_buffer_rsrc_t ors = partials_rsrc(p);
+  for (int e = threadIdx.x; e < rows * (kD / 4); e += threads) {
+    const int row = e / (kD / 4), d0 = e % (kD / 4) * 4;
+    const int64_t base = pair * kResidues * p.rows_alloc + row;
+    float2 ml[kResidues];
+    f32x4 os[kResidues];
+#pragma unroll
+    for (int r = 0; r < kResidues; ++r) {
+      const int64_t b = base + (int64_t)r * p.rows_alloc;
+      ml[r] = __builtin_bit_cast(float2, __hip_atomic_load((const uint64_t*)(p.part_ml + b * 2), __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_AGENT));
+      os[r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                            ors, (uint32_t)((b * kD + d0) * sizeof(float)), 0, kCpolAgent));
+    }
+    float M = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < kResidues; ++r) M = fmaxf(M, ml[r].x);
+    float L = 0.f;
+    f32x4 acc = f32x4{};
+#pragma unroll
+    for (int r = 0; r < kResidues; ++r) {
+      const float f = merge_scale(ml[r].x, M);
+      L = __builtin_fmaf(ml[r].y, f, L);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(os[r][i], f, acc[i]);
+    }
+    const int i = it.p0 + row / p.g;
+    const int hq = h * p.g + row % p.g;
+    uint2 w;
+    w.x = cvt_bf16x2(L == 0.f ? 0.f : acc[0] / L, L == 0.f ? 0.f : acc[1] / L);
+    w.y = cvt_bf16x2(L == 0.f ? 0.f : acc[2] / L, L == 0.f ? 0.f : acc[3] / L);
+    *(uint2*)(p.out + (int64_t)(it.q_start + i) * p.out_stride + hq * kD + d0) = w;
+  }
 }
 
 // One (item, KV head h) with the workgroup's kWaves waves, owning residues bx*kWaves .. +kWaves-1; `lds`
@@ -692,19 +774,18 @@ __device__ __forceinline__ void attn_body(const Params& p, uint8_t* lds, int ite
   if constexpr (kDeep) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
   if constexpr (!kMergeHere) {
-    // ---- write this residue's partial; attn_combine merges the eight ----
+    // ---- write this residue's partial; the pair's last workgroup or attn_combine merges the eight ----
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const int row = rt * 16 + r16;
       if (row >= rows) continue;
       const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
-      float* po = p.part_o + base * kD + 4 * grp;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) *(f32x4*)(po + 16 * dt) = o[dt][rt];
-      if (grp == 0) {
-        p.part_ml[base * 2 + 0] = m[rt];
-        p.part_ml[base * 2 + 1] = l[rt];
-      }
+      for (int dt = 0; dt < 8; ++dt) store_partial<!kVarlen && RT <= 3>(p, base, 16 * dt + 4 * grp, o[dt][rt]);
+      if (grp == 0) store_max_sum<!kVarlen && RT <= 3>(p, base, m[rt], l[rt]);
+    }
+    if constexpr (!kVarlen && RT <= 3) {
+      if (p.arrivals) merge_last(p, lds, it, item, h, kResidues / kWaves, kWaves * kWave);
     }
     return;
   } else {
@@ -877,6 +958,7 @@ __device__ __forceinline__ void stream_body(const Params& p, uint8_t* lds, int i
   auto slot_k = [&](int s) { return lds + (s % 2) * kSlotBytes; };
   auto slot_v = [&](int s) { return lds + (s % 2) * kSlotBytes + kVBuf; };
 
+  const bool merge = !kVarlen && RT <= 3 && p.arrivals;  // uniform
   if (loader) {
     // ---- the streaming wave: K in the math waves' register layout (key 16*kt + r16, d = 32*ks + 8*grp + e;
     // keys past the tile's end read its first key), V in the residue body's LDS layout ----
@@ -940,6 +1022,7 @@ __device__ __forceinline__ void stream_body(const Params& p, uint8_t* lds, int i
       load(s + 6, ra);
       prefill::block_sync();
     }
+    if (merge) merge_last(p, lds, it, item, h, kResidues, kStreamThreads);
     return;
   }
 
@@ -1040,16 +1123,14 @@ __device__ __forceinline__ void stream_body(const Params& p, uint8_t* lds, int i
     prefill::block_sync();  // this slot is free again; the next tile is in the other one
   }
 
-  // ---- this residue's partial (this wave's rows and d range); attn_combine merges the eight ----
-  if (idle || row >= rows) return;
-  const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
-  float* po = p.part_o + base * kD + 4 * grp;
+  // ---- this residue's partial (this wave's rows and d range); the last workgroup or attn_combine merges ----
+  if (!idle && row < rows) {
+    const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
 #pragma unroll
-  for (int d = 0; d < DT; ++d) *(f32x4*)(po + 16 * (dt0 + d)) = o[d];
-  if (grp == 0 && dt0 == 0) {
-    p.part_ml[base * 2 + 0] = m;
-    p.part_ml[base * 2 + 1] = l;
+    for (int d = 0; d < DT; ++d) store_partial<!kVarlen && RT <= 3>(p, base, 16 * (dt0 + d) + 4 * grp, o[d]);
+    if (grp == 0 && dt0 == 0) store_max_sum<!kVarlen && RT <= 3>(p, base, m, l);
   }
+  if (merge) merge_last(p, lds, it, item, h, kResidues, kStreamThreads);
 }
 
 template <int RT, bool kVarlen, bool kPaged>
@@ -1292,11 +1373,13 @@ __global__ __launch_bounds__(kPlanThreads) void varlen_plan(const int32_t* __res
 // (non-temporal K / V loads) when the contexts are balanced, longest at most twice the mean, so that the call
 // stays bandwidth-bound to its end; 0 when a few long contexts would leave a latency-bound tail.
 __global__ __launch_bounds__(kPlanThreads) void decode_plan(const int32_t* __restrict__ context_lens, int32_t num_seqs,
-                                                            int32_t* __restrict__ order) {
+                                                            int32_t* __restrict__ order,
+                                                            int32_t* __restrict__ arrivals, int32_t num_arrivals) {
   __shared__ uint32_t keys[kPlanThreads];
   __shared__ int64_t wsum[kPlanThreads / kWave];
   __shared__ int32_t wmax[kPlanThreads / kWave];
   const int tid = threadIdx.x;
+  for (int i = tid; i < num_arrivals; i += kPlanThreads) arrivals[i] = 0;
   if (num_seqs > kPlanThreads) {
     for (int i = tid; i < num_seqs; i += kPlanThreads) order[i] = i;
     if (tid == 0) order[num_seqs] = 1;
@@ -1342,13 +1425,14 @@ int wave_slots(hipStream_t stream) { return cu_count(stream); }
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 struct Layout {
-  size_t part_o, part_ml, work, count, work_pre, count_pre, order, total;
+  size_t part_o, part_ml, work, count, work_pre, count_pre, order, arrivals, total;
 };
 
-// Workspace: residue partials only when the merge runs in attn_combine (few items); for varlen, the two
-// work lists and their counts.
+// Workspace: residue partials only when a pair's residues span several workgroups (few items); for varlen, the
+// two work lists and their counts; for a planned decode call, the order and, with partials, the arrival counts of
+// the pairs (merge_last).
 Layout workspace_layout(int64_t items, int Hkv, int rows_alloc, bool partials, bool varlen, int64_t pre_items = 0,
-                        int64_t order_len = 0) {
+                        int64_t order_len = 0, bool arrivals = false) {
   Layout L;
   const int64_t cells = partials ? items * Hkv * kResidues * rows_alloc : 0;
   L.part_o = 0;
@@ -1358,7 +1442,8 @@ Layout workspace_layout(int64_t items, int Hkv, int rows_alloc, bool partials, b
   L.work_pre = align256(L.count + (varlen ? sizeof(int32_t) : 0));
   L.count_pre = align256(L.work_pre + (varlen ? (size_t)pre_items * 2 * sizeof(int32_t) : 0));
   L.order = align256(L.count_pre + (varlen ? 2 * sizeof(int32_t) : 0));  // all q-blocks, those with keys
-  L.total = align256(L.order + (size_t)(order_len ? order_len + 1 : 0) * sizeof(int32_t));  // + load-policy flag
+  L.arrivals = align256(L.order + (size_t)(order_len ? order_len + 1 : 0) * sizeof(int32_t));  // + load-policy flag
+  L.total = align256(L.arrivals + (arrivals ? (size_t)items * Hkv * sizeof(int32_t) : 0));
   return L;
 }
 
@@ -1382,7 +1467,7 @@ static_assert(kVarlenRT == 2, "mixed_fwd runs the residue body with two row tile
 
 // Waves per workgroup: all eight residues in one workgroup (merge in LDS) when there are enough
 // (item, head) pairs to fill the GPU and the per-wave state allows two waves per SIMD; otherwise fewer
-// residues per workgroup and more workgroups, with the merge in attn_combine.
+// residues per workgroup and more workgroups, with the merge after them.
 int residue_waves(int64_t items, int Hkv, int RT) {
   const int64_t pairs = items * Hkv;
   if (RT <= 3 && pairs >= 256) return 8;
@@ -1390,6 +1475,12 @@ int residue_waves(int64_t items, int Hkv, int RT) {
   if (pairs >= 32) return 2;
   return 1;
 }
+
+// Decode calls whose partials the pair's last workgroup may merge (merge_last): those with a plan, which clears the
+// arrival counts, and up to three row tiles, i.e. under 256 pairs (four tiles have partials at any size, and 64
+// rows are more than one workgroup should merge). The others run attn_combine. The partials' byte offsets fit 31 bits:
+// 255 pairs x 8 residues x 48 rows x 512 B = 50 MB.
+bool merges_last(bool partials, int RT) { return partials && RT <= 3; }
 
 int check_heads(const char* who, int Hq, int Hkv, int D) {
   if (D != kD) return fail(kUnsupported, "%s: head_dim %d not supported (only %d)", who, D, kD);
@@ -1448,7 +1539,7 @@ extern "C" size_t sd_paged_decode_workspace_size(int32_t num_seqs, int32_t num_q
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
   const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
-  return workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs).total;
+  return workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, merges_last(partials, RT)).total;
 }
 
 namespace {
@@ -1482,7 +1573,8 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   if (items > 65535) return fail(kUnsupported, "%s: %lld work items exceed the grid limit", who, (long long)items);
   const int waves = residue_waves(items, num_kv_heads, RT);
   const bool partials = waves < kResidues;
-  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs);
+  const bool last = merges_last(partials, RT);
+  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   // The unplanned call needs the workspace only for partials; the planned one reads the order from it.
   const size_t need = planned ? lay.total : partials ? lay.order : 0;
   if (need && (!workspace || workspace_bytes < need))
@@ -1515,11 +1607,12 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   p.part_ml = partials ? (float*)((uint8_t*)workspace + lay.part_ml) : nullptr;
   p.seq_order = planned ? (const int32_t*)((uint8_t*)workspace + lay.order) : nullptr;
   p.stream_flag = planned ? p.seq_order + num_seqs : nullptr;
+  p.arrivals = planned && last ? (int32_t*)((uint8_t*)workspace + lay.arrivals) : nullptr;
 
   hipStream_t s = (hipStream_t)stream;
   launch_fwd<false, true>(RT, waves, dim3(1, num_kv_heads, (unsigned)items), s, p);
   if ((rc = check_launch(who))) return rc;
-  if (partials) {
+  if (partials && !p.arrivals) {
     // Four rows a workgroup over the rows a query group can hold (P positions x g heads), not the row tiles'
     // padding: B=16, k=4 merges 20 of 32 rows.
     const int merge_rows = std::min(P * g, p.rows_alloc);
@@ -1566,11 +1659,13 @@ extern "C" int sd_paged_decode_plan(const int32_t* context_lens, int32_t num_seq
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
   const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
-  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs);
+  const bool last = merges_last(partials, RT);
+  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   if (!workspace || workspace_bytes < lay.total)
     return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B", who, workspace_bytes, lay.total);
   hipLaunchKernelGGL(decode_plan, dim3(1), dim3(kPlanThreads), 0, (hipStream_t)stream, context_lens, num_seqs,
-                     (int32_t*)((uint8_t*)workspace + lay.order));
+                     (int32_t*)((uint8_t*)workspace + lay.order), (int32_t*)((uint8_t*)workspace + lay.arrivals),
+                     last ? (int32_t)(items * num_kv_heads) : 0);
   return check_launch(who);
 }
 

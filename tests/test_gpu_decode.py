@@ -218,6 +218,24 @@ def test_planned_few_pairs_equals_unplanned_bitwise(device, B, n):
         assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
 
 
+@pytest.mark.parametrize("B,n,Hq,Hkv", [(1, 2, 8, 1), (10, 5, 12, 3), (15, 9, 32, 8), (31, 5, 16, 8), (127, 3, 14, 2)])
+def test_planned_last_workgroup_merge_bitwise(device, B, n, Hq, Hkv):
+    """The pair's last workgroup merges the partials (planned calls with few pairs: eight, four or two workgroups a
+    pair, 8 to 36 rows): bitwise the unplanned call's attn_combine, on six layers that share a plan and its
+    arrival counts back to back."""
+    from types import SimpleNamespace
+    rnd = random.Random(B * 10 + n)
+    ctx = [rnd.randint(0, 1200) for _ in range(B)]
+    lens = torch.tensor(ctx, dtype=torch.int32, device=device)
+    owner = SimpleNamespace()
+    kc, vc, tables = paged_cache(device, ctx, Hkv, 128, W=5, seed=400)
+    qs = [queries(device, B * n, Hq, 128, seed=401 + i).view(B, n, Hq, 128) for i in range(6)]
+    refs = [paged_decode_attention(q, kc, vc, lens, tables, 128 ** -0.5) for q in qs]
+    outs = [paged_decode_attention(q, kc, vc, lens, tables, 128 ** -0.5, plan_owner=owner) for q in qs]
+    for i in range(6):
+        assert torch.equal(outs[i], refs[i]), i
+
+
 def test_planned_past_1024_sequences(device):
     """1100 sequences, more than the plan's 1024-thread sort (the dispatch order is then the index order, and
     the plan's scan takes two passes): the planned call equals the unplanned one bitwise, and a sample of
