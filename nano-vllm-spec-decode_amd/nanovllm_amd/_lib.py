@@ -63,6 +63,10 @@ SIGNATURES = {
     "sd_sample": (_i32, [_c_void_p, _i32, _i64, _c_void_p, _c_void_p, _i32, _i32, _c_void_p, _c_void_p, _size,
                          _c_void_p]),
 }
+# Kernels of this package's own layers, not part of the C ABI.
+INTERNAL = {
+    "sd_silu_mul": (_i32, [_c_void_p, _i64, _i32, _i32, _c_void_p, _i64, _c_void_p]),
+}
 
 _lib = None
 
@@ -75,7 +79,7 @@ def load() -> ctypes.CDLL:
             raise RuntimeError(f"HIP extension not built: {LIB_PATH} is missing "
                                "(run `python nano-vllm-spec-decode_amd/build_ext.py`)")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **INTERNAL}.items():
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args

@@ -15,8 +15,8 @@ on each token alone (no step metadata), so one recording serves every step padde
 The norms follow the reference's RMSNorm arithmetic (nanovllm/layers/layernorm.py:16-38: fp32 mean of squares,
 rsqrt, cast, times the weight); the GEMMs are torch's (hipBLASLt).
 
-row_invariant=True runs the projections through RowInvariantLinear (sd_linear) and the norms through
-sd_rms_norm instead: every op then computes a token's row the same way whatever the step's token count, so a
+row_invariant=True runs the projections through RowInvariantLinear (sd_linear), the norms through sd_rms_norm
+(which update the residual in place) and the activation through sd_silu_mul instead: every op then computes a token's row the same way whatever the step's token count, so a
 token's hidden state, and the greedy token picked from it, do not depend on the batch. That is what makes
 greedy speculative decoding (1 + k rows per sequence) pick exactly the tokens of plain decoding (one row); with
 the library GEMMs and reductions, whose kernels change with the row count, near-ties can flip.
@@ -27,6 +27,7 @@ import torch
 import torch.nn.functional as F
 
 from nanovllm_amd.layers import layernorm
+from nanovllm_amd.layers.activation import silu_and_mul
 from nanovllm_amd.layers.linear import RowInvariantLinear
 from nanovllm_amd.layers.rotary_embedding import RotaryEmbedding
 
@@ -97,16 +98,23 @@ class Qwen3Segments:
             return F.linear(x, w[name])
         return torch.mm(x, w[name].t(), out=out)
 
-    def _norm(self, x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor | None = None):
-        if self.row_invariant:
-            return layernorm.rms_norm(x, weight, self.eps, residual)
-        return rms_norm(x, weight, self.eps) if residual is None else add_rms_norm(x, residual, weight, self.eps)
+    def _norm(self, x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor | None = None,
+              out: torch.Tensor | None = None):
+        if self.row_invariant:   # the residual is updated in place
+            return layernorm.rms_norm(x, weight, self.eps, residual, out=out, residual_out=residual)
+        res = rms_norm(x, weight, self.eps) if residual is None else add_rms_norm(x, residual, weight, self.eps)
+        if out is not None:
+            out.copy_(res if residual is None else res[0])
+        return res
 
     def _post_attn(self, w: dict, o: torch.Tensor, residual: torch.Tensor):
         """Qwen3DecoderLayer.post_attn (qwen3.py:192-201)."""
         h = self._linear(o, w, "o")
         h, residual = self._norm(h, w["post_norm"], residual)
-        gate, up = self._linear(h, w, "gate_up").chunk(2, -1)
+        h = self._linear(h, w, "gate_up")
+        if self.row_invariant:
+            return self._linear(silu_and_mul(h), w, "down"), residual
+        gate, up = h.chunk(2, -1)
         return self._linear(F.silu(gate) * up, w, "down"), residual
 
     def __call__(self, i: int, n: int, bufs: dict) -> None:
@@ -116,8 +124,9 @@ class Qwen3Segments:
         else:
             h, residual = self._post_attn(self.layers[i - 1], bufs["o"][:n].view(n, -1), self.residual[:n])
             if i == self.L:
-                self.hidden_out[:n] = self._norm(h, self.final_norm, residual)[0]
+                self._norm(h, self.final_norm, residual, out=self.hidden_out[:n])
                 return
             x, residual = self._norm(h, self.layers[i]["in_norm"], residual)
-        self.residual[:n] = residual
+        if i == 0 or not self.row_invariant:
+            self.residual[:n] = residual
         self._linear(x, self.layers[i], "qkv", out=bufs["qkv"][:n])

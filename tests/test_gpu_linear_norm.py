@@ -10,6 +10,7 @@ library GEMM (o_proj, gate_up_proj and down_proj shapes) and reductions do not.
 import pytest
 import torch
 
+from nanovllm_amd.layers.activation import silu_and_mul
 from nanovllm_amd.layers.layernorm import RMSNorm, rms_norm
 from nanovllm_amd.layers.linear import RowInvariantLinear
 from oracle import qk_norm_rope as onr
@@ -144,3 +145,21 @@ def test_linear_output_over_its_input(device):
         x = torch.randn(M, 512, device=device, generator=g).to(torch.bfloat16)
         want = lin(x)
         assert torch.equal(lin(x, out=x), want)
+
+
+# SiLU-and-multiply against the eager operations in float64 with their two roundings: the fp32 silu is within a few
+# units of 2^-24, so its bf16 rounding moves by at most one unit and only where it lies that close to a midpoint.
+@pytest.mark.parametrize("M,half", [(1, 8), (5, 2056), (80, 12288), (3, 2048)])
+def test_silu_and_mul(device, M, half):
+    g = torch.Generator(device=device).manual_seed(half)
+    wide = (4 * torch.randn(M, 2 * half + 8, device=device, generator=g)).to(torch.bfloat16)
+    x = wide[:, :2 * half]                                    # a row stride past the row
+    x[0, :6] = torch.tensor([0.0, -0.0, 200.0, -200.0, float("inf"), float("nan")])
+    gate, up = x.double().chunk(2, -1)
+    want = ((gate / (1 + torch.exp(-gate))).to(torch.bfloat16).double() * up).to(torch.bfloat16)
+    got = silu_and_mul(x)
+    ok = (got.view(torch.int16) == want.view(torch.int16)) | (got.isnan() & want.isnan()) | (got == want)
+    assert ok.float().mean().item() >= 0.999
+    finite = want.isfinite()
+    assert bool(((got.float() - want.float()).abs()[finite] <= 2 * _ulp_bf16(want.float())[finite]).all())
+    assert torch.equal(silu_and_mul(x[:1])[0].view(torch.int16), got[0].view(torch.int16))
