@@ -197,9 +197,10 @@ __device__ __forceinline__ float merge_scale(float m_r, float M) {
   return exp2_fast(m_r - (M == -INFINITY ? 0.f : M));
 }
 
-// A residue's partials. kThrough: decode calls that merge_last may finish, whose workgroups run on several XCDs with
+// A residue's partials. kThrough: calls that merge_last finishes, whose workgroups run on several XCDs with
 // an L2 each: stores at agent scope (written through) and loads at agent scope, so that no fence has to write back or
-// drop an L2. With release and acquire fences instead, B=1 took 14.3 us a layer, against 12.7 with attn_combine.
+// drop an L2. With release and acquire fences instead, B=1 took 14.3 us a layer, against 12.7 with attn_combine. In
+// front of attn_combine they cost instead (B=16, k=4, 2000 keys without a plan: 31.9 us against 31.3).
 constexpr int kCpolAgent = 16;  // sc1
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t partials_rsrc(const Params& p) {
   return __builtin_amdgcn_make_buffer_rsrc(p.part_o, 0, 0x7fffffff, 0x00020000);
@@ -775,18 +776,26 @@ __device__ __forceinline__ void attn_body(const Params& p, uint8_t* lds, int ite
 
   if constexpr (!kMergeHere) {
     // ---- write this residue's partial; the pair's last workgroup or attn_combine merges the eight ----
+    auto store = [&](auto through) __attribute__((always_inline)) {
+      constexpr bool kThrough = decltype(through)::value;
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) {
-      const int row = rt * 16 + r16;
-      if (row >= rows) continue;
-      const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
+      for (int rt = 0; rt < RT; ++rt) {
+        const int row = rt * 16 + r16;
+        if (row >= rows) continue;
+        const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
 #pragma unroll
-      for (int dt = 0; dt < 8; ++dt) store_partial<!kVarlen && RT <= 3>(p, base, 16 * dt + 4 * grp, o[dt][rt]);
-      if (grp == 0) store_max_sum<!kVarlen && RT <= 3>(p, base, m[rt], l[rt]);
-    }
+        for (int dt = 0; dt < 8; ++dt) store_partial<kThrough>(p, base, 16 * dt + 4 * grp, o[dt][rt]);
+        if (grp == 0) store_max_sum<kThrough>(p, base, m[rt], l[rt]);
+      }
+    };
     if constexpr (!kVarlen && RT <= 3) {
-      if (p.arrivals) merge_last(p, lds, it, item, h, kResidues / kWaves, kWaves * kWave);
+      if (p.arrivals) {  // uniform
+        store(std::true_type{});
+        merge_last(p, lds, it, item, h, kResidues / kWaves, kWaves * kWave);
+        return;
+      }
     }
+    store(std::false_type{});
     return;
   } else {
     // ---- merge the eight residues in order: every wave parks its O in LDS, then each thread finishes
@@ -1124,11 +1133,18 @@ __device__ __forceinline__ void stream_body(const Params& p, uint8_t* lds, int i
   }
 
   // ---- this residue's partial (this wave's rows and d range); the last workgroup or attn_combine merges ----
-  if (!idle && row < rows) {
+  auto store_rows = [&](auto through) __attribute__((always_inline)) {
+    constexpr bool kThrough = decltype(through)::value;
     const int64_t base = (((int64_t)item * p.Hkv + h) * kResidues + residue) * p.rows_alloc + row;
 #pragma unroll
-    for (int d = 0; d < DT; ++d) store_partial<!kVarlen && RT <= 3>(p, base, 16 * (dt0 + d) + 4 * grp, o[d]);
-    if (grp == 0 && dt0 == 0) store_max_sum<!kVarlen && RT <= 3>(p, base, m, l);
+    for (int d = 0; d < DT; ++d) store_partial<kThrough>(p, base, 16 * (dt0 + d) + 4 * grp, o[d]);
+    if (grp == 0 && dt0 == 0) store_max_sum<kThrough>(p, base, m, l);
+  };
+  if (!idle && row < rows) {
+    if (merge)
+      store_rows(std::true_type{});
+    else
+      store_rows(std::false_type{});
   }
   if (merge) merge_last(p, lds, it, item, h, kResidues, kStreamThreads);
 }
