@@ -866,7 +866,8 @@ __device__ __forceinline__ void attn_body(const Params& p, uint8_t* lds, int ite
 // therefore rotated by one per batch of workgroups the GPU holds at once: an XCD runs one head at a
 // time, a different one in each such batch (B=64 k=4: 193.7 -> 180.8 us).
 __device__ __forceinline__ int rotated_head(const Params& p, int y, int z) {
-  const int64_t linear = ((int64_t)z * gridDim.y + y) * gridDim.x;
+  // by the item's first workgroup, so that an item's heads are a rotation whatever their number
+  const int64_t linear = (int64_t)z * gridDim.y * gridDim.x;
   return (int)((y + linear / p.wave_slots) % p.Hkv);
 }
 
@@ -1174,8 +1175,8 @@ template <bool kPaged, int kPreRowGroups, int kPreStageTiles>
 __global__ __launch_bounds__(kResidues * kWave, 2) void mixed_fwd(Params p, PrefillArgs a) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[kMixedLds];
   // KV head fastest along the grid, rotated by one per batch of resident workgroups (see rotated_head).
-  const int h = (int)((blockIdx.x % a.Hkv + blockIdx.x / p.wave_slots) % a.Hkv);
   const int x = blockIdx.x / a.Hkv;
+  const int h = (int)((blockIdx.x % a.Hkv + (blockIdx.x - blockIdx.x % a.Hkv) / p.wave_slots) % a.Hkv);
   // The plan's counts (each at most its grid share): np prefill q-blocks, the first npk of them from sequences
   // with keys (the rest see no key: a padded bucket's padding rows, which only write zeros), nr residue items.
   const int np = a.work_count[0], npk = a.work_count[1], nr = *p.work_count;

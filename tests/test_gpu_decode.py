@@ -10,7 +10,7 @@ import random
 import pytest
 import torch
 
-from nanovllm_amd.layers.attention import paged_decode_attention
+from nanovllm_amd.layers.attention import paged_decode_attention, varlen_attention
 from oracle import attention as oatt
 from attn_cases import error_stats, paged_cache, queries, sub_cache
 
@@ -216,6 +216,29 @@ def test_planned_few_pairs_equals_unplanned_bitwise(device, B, n):
         o = oatt.paged_decode_attention(q.cpu(), kc.cpu(), vc.cpu(), lens.cpu(), tables.cpu(), 128 ** -0.5)
         mx, mean = error_stats(fused.view(B, n, 32, 128), o)
         assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
+
+
+@pytest.mark.parametrize("B,n,Hq,Hkv", [(10, 1, 21, 7), (40, 5, 28, 7), (100, 2, 12, 3), (37, 17, 10, 5)])
+def test_kv_head_counts_that_do_not_divide_the_cus(device, B, n, Hq, Hkv):
+    """The KV head rotation of a batch of workgroups may change inside an item's heads: every head is computed once
+    (3, 5 and 7 KV heads; two, four and eight waves a workgroup and the varlen launch with q-blocks)."""
+    rnd = random.Random(B + n)
+    ctx = [rnd.randint(n, 400) for _ in range(B)]
+    kc, vc, tables = paged_cache(device, ctx, Hkv, 128, seed=500)
+    q = queries(device, B * n, Hq, 128, seed=501)
+    lens = torch.tensor(ctx, dtype=torch.int32, device=device)
+    if n <= 16:
+        out = paged_decode_attention(q.view(B, n, Hq, 128), kc, vc, lens, tables, 128 ** -0.5)
+        ref = oatt.paged_decode_attention(q.view(B, n, Hq, 128).cpu(), kc.cpu(), vc.cpu(), lens.cpu(), tables.cpu(),
+                                          128 ** -0.5)
+        mx, mean = error_stats(out.view(B, n, Hq, 128), ref)
+    else:
+        cu_q = torch.arange(0, B * n + 1, n, dtype=torch.int32, device=device)
+        cu_k = torch.cat([lens.new_zeros(1), lens.cumsum(0, dtype=torch.int32)])
+        out = varlen_attention(q, kc, vc, cu_q, cu_k, n, max(ctx), 128 ** -0.5, tables)
+        ref = oatt.varlen_attention(q.cpu(), kc.cpu(), vc.cpu(), cu_q.cpu(), cu_k.cpu(), 128 ** -0.5, tables.cpu())
+        mx, mean = error_stats(out, ref)
+    assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
 
 
 @pytest.mark.parametrize("B,n,Hq,Hkv", [(1, 2, 8, 1), (10, 5, 12, 3), (15, 9, 32, 8), (31, 5, 16, 8), (127, 3, 14, 2)])
