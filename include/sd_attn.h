@@ -116,8 +116,9 @@ int sd_paged_decode(const void* q, int64_t q_token_stride, const void* k_cache, 
  * the mean), the default policy otherwise; sd_paged_decode always loads non-temporal. Order and policy only
  * decide which workgroup computes which sequence and how it loads: results are bitwise those of
  * sd_paged_decode even when the plan was made for other context lengths, as long as it was made for the
- * same num_seqs. With too few pairs to merge inside one workgroup, the planned call's last workgroup of a pair
- * merges its partials (the plan clears the arrival counts in the workspace, each call leaves them cleared).
+ * same num_seqs. With too few pairs to merge inside one workgroup and few rows a pair, the planned call's last
+ * workgroup of a pair merges its partials (the plan clears the arrival counts in the workspace, each call leaves
+ * them cleared).
  * No counterpart in the reference; it serves the per-layer loop of a decode step
  * (nanovllm/engine/model_runner.py:476-485).
  */

@@ -111,7 +111,7 @@ struct Params {
   int64_t out_stride;
   float* part_o;                // [item][Hkv][kResidues][rows_alloc][kD]
   float* part_ml;               // [item][Hkv][kResidues][rows_alloc][2] = (max, sum)
-  int32_t* arrivals;            // [item][Hkv] workgroups of the pair that are done, or null: attn_combine merges
+  int32_t* arrivals;            // [item][Hkv] workgroups of the pair that are done; null: attn_combine merges
   int32_t wave_slots;           // workgroups the GPU runs at once (one per CU): the head rotation period
 };
 
@@ -227,8 +227,8 @@ __device__ __forceinline__ void store_max_sum(const Params& p, int64_t cell, flo
 // `wgs` workgroups to come here merges the eight partials and writes the pair's rows; `lds` is free. Every wave waits
 // for its stores before the workgroup arrives. The arrival count is 0 between launches: the plan clears it and the
 // last workgroup resets it. The merge as a kernel of its own took 3.9-4.8 us and its launch; here it is one round trip
-// for the arrival and one for the partials (8 layers of B=1, 1500 keys: 102 -> 94-96 us; 4 layers of B=16, k=4: 199 ->
-// 197). Each thread finishes four consecutive d of one row, with attn_combine's fma chain.
+// for the arrival and one for the partials (8 layers of B=1, 1500 keys: 102 -> 94-96 us). Each thread finishes four
+// consecutive d of one row, with attn_combine's fma chain.
 __device__ __forceinline__ void merge_last(const Params& p, uint8_t* lds, const Item& it, int item, int h, int wgs,
                                            int threads) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's partials are stored
@@ -788,7 +788,7 @@ __device__ __forceinline__ void attn_body(const Params& p, uint8_t* lds, int ite
         if (grp == 0) store_max_sum<kThrough>(p, base, m[rt], l[rt]);
       }
     };
-    if constexpr (!kVarlen && RT <= 3) {
+    if constexpr (!kVarlen && RT == 1) {
       if (p.arrivals) {  // uniform
         store(std::true_type{});
         merge_last(p, lds, it, item, h, kResidues / kWaves, kWaves * kWave);
@@ -968,7 +968,7 @@ __device__ __forceinline__ void stream_body(const Params& p, uint8_t* lds, int i
   auto slot_k = [&](int s) { return lds + (s % 2) * kSlotBytes; };
   auto slot_v = [&](int s) { return lds + (s % 2) * kSlotBytes + kVBuf; };
 
-  const bool merge = !kVarlen && RT <= 3 && p.arrivals;  // uniform
+  const bool merge = !kVarlen && RT == 1 && p.arrivals;  // uniform
   if (loader) {
     // ---- the streaming wave: K in the math waves' register layout (key 16*kt + r16, d = 32*ks + 8*grp + e;
     // keys past the tile's end read its first key), V in the residue body's LDS layout ----
@@ -1493,11 +1493,16 @@ int residue_waves(int64_t items, int Hkv, int RT) {
   return 1;
 }
 
-// Decode calls whose partials the pair's last workgroup may merge (merge_last): those with a plan, which clears the
-// arrival counts, and up to three row tiles, i.e. under 256 pairs (four tiles have partials at any size, and 64
-// rows are more than one workgroup should merge). The others run attn_combine. The partials' byte offsets fit 31 bits:
-// 255 pairs x 8 residues x 48 rows x 512 B = 50 MB.
-bool merges_last(bool partials, int RT) { return partials && RT <= 3; }
+// Decode calls whose partials the pair's last workgroup merges (merge_last): those with a plan, which clears the
+// arrival counts, whose pair's rows fit one pass of the workgroup (4 columns a thread: 10 rows for the stream kernel,
+// 8 and 4 for four and two waves). The other calls run attn_combine, which spreads the rows over the GPU. Measured
+// (us a layer, attn_combine -> merge_last): 4 rows, 1 x 300 keys 8.5 -> 8.0, 16 x 300 keys 10.7 -> 10.3; more
+// than a pass: 20 rows, 1 x 4096 keys 19.5 -> 20.5, 4 x 2000 keys 18.9 -> 21.8; 36 rows, 2 x 1000 keys 11.5 -> 14.8.
+bool merges_last(int waves, int merge_rows) {
+  if (waves == kResidues) return false;
+  const int threads = waves == 1 ? kStreamThreads : waves * kWave;
+  return merge_rows * (kD / 4) <= threads;
+}
 
 int check_heads(const char* who, int Hq, int Hkv, int D) {
   if (D != kD) return fail(kUnsupported, "%s: head_dim %d not supported (only %d)", who, D, kD);
@@ -1555,8 +1560,9 @@ extern "C" size_t sd_paged_decode_workspace_size(int32_t num_seqs, int32_t num_q
   int RT, P;
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
-  const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
-  return workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, merges_last(partials, RT)).total;
+  const int waves = residue_waves(items, num_kv_heads, RT);
+  const bool last = merges_last(waves, std::min(P * (num_heads / num_kv_heads), RT * 16));
+  return workspace_layout(items, num_kv_heads, RT * 16, waves < kResidues, false, 0, num_seqs, last).total;
 }
 
 namespace {
@@ -1590,7 +1596,8 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   if (items > 65535) return fail(kUnsupported, "%s: %lld work items exceed the grid limit", who, (long long)items);
   const int waves = residue_waves(items, num_kv_heads, RT);
   const bool partials = waves < kResidues;
-  const bool last = merges_last(partials, RT);
+  const int merge_rows = std::min(P * g, RT * 16);  // rows a query group can hold, not the row tiles' padding
+  const bool last = merges_last(waves, merge_rows);
   const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   // The unplanned call needs the workspace only for partials; the planned one reads the order from it.
   const size_t need = planned ? lay.total : partials ? lay.order : 0;
@@ -1630,9 +1637,7 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   launch_fwd<false, true>(RT, waves, dim3(1, num_kv_heads, (unsigned)items), s, p);
   if ((rc = check_launch(who))) return rc;
   if (partials && !p.arrivals) {
-    // Four rows a workgroup over the rows a query group can hold (P positions x g heads), not the row tiles'
-    // padding: B=16, k=4 merges 20 of 32 rows.
-    const int merge_rows = std::min(P * g, p.rows_alloc);
+    // Four rows a workgroup: B=16, k=4 merges 20 of 32 rows.
     hipLaunchKernelGGL((attn_combine<false>), dim3((unsigned)items, num_kv_heads, (unsigned)((merge_rows + 3) / 4)),
                        dim3(256), 0, s, p);
     if ((rc = check_launch(who))) return rc;
@@ -1675,8 +1680,9 @@ extern "C" int sd_paged_decode_plan(const int32_t* context_lens, int32_t num_seq
   int RT, P;
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
-  const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
-  const bool last = merges_last(partials, RT);
+  const int waves = residue_waves(items, num_kv_heads, RT);
+  const bool partials = waves < kResidues;
+  const bool last = merges_last(waves, std::min(P * (num_heads / num_kv_heads), RT * 16));
   const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   if (!workspace || workspace_bytes < lay.total)
     return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B", who, workspace_bytes, lay.total);
