@@ -788,7 +788,7 @@ __device__ __forceinline__ void attn_body(const Params& p, uint8_t* lds, int ite
         if (grp == 0) store_max_sum<kThrough>(p, base, m[rt], l[rt]);
       }
     };
-    if constexpr (!kVarlen && RT == 1) {
+    if constexpr (!kVarlen && RT == 1 && kWaves == 4) {
       if (p.arrivals) {  // uniform
         store(std::true_type{});
         merge_last(p, lds, it, item, h, kResidues / kWaves, kWaves * kWave);
@@ -1495,13 +1495,14 @@ int residue_waves(int64_t items, int Hkv, int RT) {
 
 // Decode calls whose partials the pair's last workgroup merges (merge_last): those with a plan, which clears the
 // arrival counts, whose pair's rows fit one pass of the workgroup (4 columns a thread: 10 rows for the stream kernel,
-// 8 and 4 for four and two waves). The other calls run attn_combine, which spreads the rows over the GPU. Measured
-// (us a layer, attn_combine -> merge_last): 4 rows, 1 x 300 keys 8.5 -> 8.0, 16 x 300 keys 10.7 -> 10.3; more
-// than a pass: 20 rows, 1 x 4096 keys 19.5 -> 20.5, 4 x 2000 keys 18.9 -> 21.8; 36 rows, 2 x 1000 keys 11.5 -> 14.8.
-bool merges_last(int waves, int merge_rows) {
-  if (waves == kResidues) return false;
+// 8 for four waves), at most 8 pairs or from 128 on (four waves). The other calls run attn_combine, which spreads the
+// rows over the GPU. Measured (us a layer, attn_combine -> merge_last, 8 KV heads): 4 rows, 1 x 300 keys 8.5 -> 8.0,
+// 1 x 4096 19.9 -> 19.3, 16 x 300 10.8 -> 10.4; 8 rows, 16 x 300 11.9 -> 10.9; between, 4 rows, 2 x 1000 10.1 ->
+// 10.8, 3 x 2000 the same, 8 x 300 9.1 -> 9.5; more than a pass: 20 rows, 1 x 4096 19.5 -> 20.5, 4 x 2000
+// 18.9 -> 21.8; 36 rows, 2 x 1000 11.5 -> 14.8.
+bool merges_last(int waves, int64_t pairs, int merge_rows) {
   const int threads = waves == 1 ? kStreamThreads : waves * kWave;
-  return merge_rows * (kD / 4) <= threads;
+  return (waves == 4 || (waves == 1 && pairs <= 8)) && merge_rows * (kD / 4) <= threads;
 }
 
 int check_heads(const char* who, int Hq, int Hkv, int D) {
@@ -1561,7 +1562,7 @@ extern "C" size_t sd_paged_decode_workspace_size(int32_t num_seqs, int32_t num_q
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
   const int waves = residue_waves(items, num_kv_heads, RT);
-  const bool last = merges_last(waves, std::min(P * (num_heads / num_kv_heads), RT * 16));
+  const bool last = merges_last(waves, items * num_kv_heads, std::min(P * (num_heads / num_kv_heads), RT * 16));
   return workspace_layout(items, num_kv_heads, RT * 16, waves < kResidues, false, 0, num_seqs, last).total;
 }
 
@@ -1597,7 +1598,7 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   const int waves = residue_waves(items, num_kv_heads, RT);
   const bool partials = waves < kResidues;
   const int merge_rows = std::min(P * g, RT * 16);  // rows a query group can hold, not the row tiles' padding
-  const bool last = merges_last(waves, merge_rows);
+  const bool last = merges_last(waves, items * num_kv_heads, merge_rows);
   const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   // The unplanned call needs the workspace only for partials; the planned one reads the order from it.
   const size_t need = planned ? lay.total : partials ? lay.order : 0;
@@ -1682,7 +1683,7 @@ extern "C" int sd_paged_decode_plan(const int32_t* context_lens, int32_t num_seq
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
   const int waves = residue_waves(items, num_kv_heads, RT);
   const bool partials = waves < kResidues;
-  const bool last = merges_last(waves, std::min(P * (num_heads / num_kv_heads), RT * 16));
+  const bool last = merges_last(waves, items * num_kv_heads, std::min(P * (num_heads / num_kv_heads), RT * 16));
   const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
   if (!workspace || workspace_bytes < lay.total)
     return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B", who, workspace_bytes, lay.total);

@@ -241,12 +241,12 @@ def test_kv_head_counts_that_do_not_divide_the_cus(device, B, n, Hq, Hkv):
     assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
 
 
-@pytest.mark.parametrize("B,n,Hq,Hkv", [(1, 1, 8, 1), (3, 5, 2, 1), (3, 3, 4, 1), (5, 2, 16, 8), (10, 1, 21, 7),
-                                        (20, 2, 32, 8), (127, 3, 4, 2), (127, 3, 6, 2)])
+@pytest.mark.parametrize("B,n,Hq,Hkv", [(1, 1, 8, 1), (3, 5, 2, 1), (8, 3, 3, 1), (9, 1, 4, 1), (3, 3, 4, 1),
+                                        (5, 2, 16, 8), (10, 1, 21, 7), (20, 2, 32, 8), (127, 3, 4, 2), (127, 3, 6, 2)])
 def test_planned_last_workgroup_merge_bitwise(device, B, n, Hq, Hkv):
-    """The pair's last workgroup merges the partials (planned calls with few pairs: eight, four or two workgroups a
-    pair, up to 10, 4 and 8 rows, and one past each): bitwise the unplanned call's attn_combine, on six layers
-    that share a plan and its arrival counts back to back."""
+    """The pair's last workgroup merges the partials (planned calls: up to 8 pairs with eight workgroups a pair and 10
+    rows, from 128 pairs with two and 8 rows; and calls past these): bitwise the unplanned call's attn_combine, on
+    six layers that share a plan and its arrival counts back to back."""
     from types import SimpleNamespace
     rnd = random.Random(B * 10 + n)
     ctx = [rnd.randint(0, 1200) for _ in range(B)]
