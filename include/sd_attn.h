@@ -213,8 +213,9 @@ int sd_verify_drafts(const void* logits, int32_t logits_dtype, int64_t logits_ro
  * stride >= vocab) is required and the sampled rows are decided by sd_verify_drafts's passes over it. The
  * other arguments and the outputs are sd_verify_drafts's. No counterpart in the reference for the packing (the
  * reference's F.linear reads the weight as stored). A token row's logits depend on its hidden row, the weight and
- * hidden_dim only, never on the call's row count (num_seqs * (K+1)) or the device's CU count: each logit is one
- * fp32 chain over hidden_dim in order, whichever kernel computes it. K = 0 is plain sampling (Sampler.forward,
+ * (vocab, hidden_dim) only, never on the call's row count (num_seqs * (K+1)) or the device's CU count: each logit is
+ * a sum in fp32 of ranges of hidden_dim in order, whichever kernel computes it; how many ranges (one, or up to 8 for
+ * the last vocabulary rows) follows from (vocab, hidden_dim) alone. K = 0 is plain sampling (Sampler.forward,
  * sampler.py:7-16, on compute_logits' rows), so plain decode and verify steps read the same logits.
  */
 size_t sd_lm_head_packed_weight_size(int32_t vocab, int32_t hidden_dim);

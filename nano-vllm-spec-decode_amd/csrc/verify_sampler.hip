@@ -940,8 +940,8 @@ __global__ __launch_bounds__(64) void lm_head_poison(const int64_t* rows, int32_
 }
 
 // The kernel a row-invariant GEMM call runs: every choice gives the same bits, so the rule looks at time alone.
-enum RowShape { kStream16, kStream32, k256x32, k32x64, k32x80, k64x80, k128x64, k128x80, k128x160, k256x128, k256x160,
-                k256x256 };
+enum RowShape { kStream16, kStream32, k256x32, k32x64E16, k32x64, k32x80, k64x80, k128x64, k128x80, k128x160, k256x128,
+                k256x160, k256x256 };
 struct RowPlan {
   RowShape shape;
   int tiles_n, tiles_m;
@@ -952,8 +952,9 @@ struct RowPlan {
 // shape with the least rounds of workgroups over the GPU x time of a workgroup, from each shape's measured time per
 // step of 32 columns (on all CUs, one workgroup each) and about 6 us of launch, first loads and epilogue, but never
 // less than the weight takes from HBM; of equal ones the first. A larger shape loads less per MFMA, a smaller one
-// keeps more CUs busy: at 320 rows 4096 x 4096 takes 26 us as 64 x 80 and 56 as 256 x 128, at 1168 rows
-// 24576 x 4096 203 us as 256 x 256 and 255 as 128 x 160.
+// keeps more CUs busy: at 320 rows 4096 x 4096 takes 25 us as 64 x 80 and 57 as 256 x 128, at 1168 rows
+// 24576 x 4096 207 us as 256 x 160 and 226 as 256 x 128. 256 x 256 has no registers for a sum of ranges: it takes
+// weights of one range a tile only (with its one-range sums 24576 x 4096 took 193 us).
 RowPlan row_plan(int M, int N, int K) {
   if (M <= lmhead::kStreamRows) {
     if (N >= 512 * lmhead::kN) return {k256x32, (N + lmhead::kN - 1) / lmhead::kN, 1};
@@ -962,19 +963,24 @@ RowPlan row_plan(int M, int N, int K) {
   }
   struct Shape {
     RowShape shape;
-    int rows_n, rows_m, step_ns;
+    int rows_n, rows_m, step_ns, ends;   // ranges end at multiples of `ends` steps (0: one range only)
   };
-  static constexpr Shape kShapes[] = {{k32x64, 32, 64, 100},     {k32x80, 32, 80, 125},     {k64x80, 64, 80, 156},
-                                      {k128x64, 128, 64, 210},   {k128x80, 128, 80, 235},   {k128x160, 128, 160, 290},
-                                      {k256x128, 256, 128, 420}, {k256x160, 256, 160, 560}, {k256x256, 256, 256, 760}};
+  static constexpr Shape kShapes[] = {
+      {k32x64E16, 32, 64, 100, 16}, {k32x64, 32, 64, 100, 1},     {k32x80, 32, 80, 125, 1},
+      {k64x80, 64, 80, 156, 1},     {k128x64, 128, 64, 210, 1},   {k128x80, 128, 80, 235, 1},
+      {k128x160, 128, 160, 290, 1}, {k256x128, 256, 128, 420, 1}, {k256x160, 256, 160, 560, 1},
+      {k256x256, 256, 256, 760, 0}};
   constexpr int kCUs = 256, kStartNs = 6000, kHbmBytesPerNs = 5600;
   const int64_t hbm_ns = (int64_t)N * K * 2 / kHbmBytesPerNs;
+  const int splits = lmhead::sum_ranges(N, K).splits, steps = K / lmhead::kK;
   RowPlan best{};
   int64_t best_ns = INT64_MAX;
   for (const Shape& c : kShapes) {
+    // the ranges' ends are multiples of `ends` if the ranges are equal and multiples themselves
+    if (splits > 1 && (c.ends == 0 || (c.ends > 1 && steps % (splits * c.ends)))) continue;
     const int tn = (N + c.rows_n - 1) / c.rows_n, tm = (M + c.rows_m - 1) / c.rows_m;
     const int64_t rounds = ((int64_t)tn * tm + kCUs - 1) / kCUs;
-    const int64_t ns = std::max(hbm_ns, rounds * ((int64_t)(K / lmhead::kK) * c.step_ns + kStartNs));
+    const int64_t ns = std::max(hbm_ns, rounds * ((int64_t)steps * c.step_ns + kStartNs));
     if (ns < best_ns) {
       best_ns = ns;
       best = {c.shape, tn, tm};
@@ -991,12 +997,16 @@ void launch_tile(const lmhead::Args& a, hipStream_t s) {
 
 int launch_row_gemm(lmhead::Args a, hipStream_t s) {
   const RowPlan p = row_plan(a.M, a.N, a.K);
+  const lmhead::Ranges ranges = lmhead::sum_ranges(a.N, a.K);
   a.tiles_n = p.tiles_n;
   a.tiles_m = p.tiles_m;
+  a.full = ranges.full;
+  a.splits = ranges.splits;
   switch (p.shape) {
     case kStream16: hipLaunchKernelGGL(lmhead::stream_gemm<1>, dim3(p.tiles_n), dim3(kWave), 0, s, a); break;
     case kStream32: hipLaunchKernelGGL(lmhead::stream_gemm<2>, dim3(p.tiles_n), dim3(kWave), 0, s, a); break;
     case k256x32: launch_tile<lmhead::Tile256x32>(a, s); break;
+    case k32x64E16: launch_tile<lmhead::Tile32x64E16>(a, s); break;
     case k32x64: launch_tile<lmhead::Tile32x64>(a, s); break;
     case k32x80: launch_tile<lmhead::Tile32x80>(a, s); break;
     case k64x80: launch_tile<lmhead::Tile64x80>(a, s); break;

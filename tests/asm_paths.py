@@ -78,3 +78,72 @@ def unsafe_asm_loads(ins, opcode="global_load_dwordx4"):
             if r:
                 bad.append((t, r))
     return bad, n
+
+
+def _all_regs(text):
+    """Vector and accumulation registers named in an instruction's operands."""
+    out = set()
+    for m in re.finditer(r"\b([va])\[(\d+):(\d+)\]", text):
+        out |= {(m.group(1), i) for i in range(int(m.group(2)), int(m.group(3)) + 1)}
+    for m in re.finditer(r"(?<![\[:\w])([va])(\d+)(?![\d:\]])", text):
+        out.add((m.group(1), int(m.group(2))))
+    return out
+
+
+def unsafe_in_flight(ins):
+    """Inline-asm loads (global_load_dwordx4 counted by vmcnt, ds_read_b128 by lgkmcnt) whose destination an
+    instruction names before a wait covers the load, over every path of the control flow graph: at each point the
+    fewest instructions of the load's counter issued after it on any path to that point. A wait for N covers a load
+    with at least N such instructions after it. Only LDS instructions count for lgkmcnt (scalar loads return out of
+    order). Returns ([(load, index, touching instruction)], global loads, LDS reads)."""
+    cap = 64
+    labels = {t.split(":")[0]: i for i, (t, _) in enumerate(ins) if re.match(r"\.L\w+:", t)}
+    ops, succ = [], []
+    for i, (t, in_asm) in enumerate(ins):
+        nxt = [i + 1] if i + 1 < len(ins) else []
+        m = re.match(r"s_(cbranch_\w+|branch)\s+(\.L\S+)", t)
+        if m:
+            succ.append([labels[m.group(2)]] + (nxt if m.group(1) != "branch" else []))
+        else:
+            assert not re.match(r"s_(setpc|swappc|call)", t), t
+            succ.append([] if t.startswith("s_endpgm") else nxt)
+        name, _, args = t.partition(" ")
+        if re.match(r"\.L\w+:", t):
+            ops.append(("none",))
+        elif name == "s_waitcnt":
+            ops.append(("wait", {k: int(n) for k, n in re.findall(r"(vmcnt|lgkmcnt)\((\d+)\)", args)}))
+        elif name.startswith("s_"):
+            ops.append(("none",))
+        else:
+            counter = "vmcnt" if _VMEM.match(t) else "lgkmcnt" if name.startswith("ds_") else None
+            load = in_asm and name in ("global_load_dwordx4", "ds_read_b128")
+            ops.append(("op", counter, _all_regs(args), _all_regs(args.split(",")[0]) if load else set()))
+    bad, state, work = {}, {0: {}}, [0]
+    while work:
+        i = work.pop()
+        cur = state[i]
+        op = ops[i]
+        if op[0] == "wait":
+            cur = {r: (c, n, j) for r, (c, n, j) in cur.items() if not (c in op[1] and n >= op[1][c])}
+        elif op[0] == "op":
+            _, counter, regs, dst = op
+            for r in regs & cur.keys():
+                bad.setdefault((cur[r][2], i), (ins[cur[r][2]][0], cur[r][2], ins[i][0]))
+            if counter:
+                cur = {r: (c, min(n + 1, cap) if c == counter else n, j) for r, (c, n, j) in cur.items()}
+                cur.update({r: (counter, 0, i) for r in dst})
+        for j in succ[i]:
+            old = state.get(j)
+            if old is None:
+                state[j] = dict(cur)
+                work.append(j)
+                continue
+            changed = False
+            for r, v in cur.items():
+                if r not in old or v[1] < old[r][1]:
+                    old[r] = v
+                    changed = True
+            if changed:
+                work.append(j)
+    n = [sum(1 for (t, a) in ins if a and t.startswith(o + " ")) for o in ("global_load_dwordx4", "ds_read_b128")]
+    return sorted(bad.values(), key=lambda x: x[1]), n[0], n[1]

@@ -1,7 +1,7 @@
 """tile_gemm issues its weight loads and LDS reads as inline asm, which the compiler does not know to be in flight.
 Compiles verify_sampler.hip (hipcc, no GPU) and checks every instantiation's gfx950 code: no destination register
-of such a load is read, copied or reused on any path before a wait that covers the load, and nothing is spilled
-(a spill could store a register whose load has not landed)."""
+of a weight load (global_load_dwordx4) or an LDS read (ds_read_b128) is read, copied or reused on any path before a
+wait that covers the load, and nothing is spilled (a spill could store a register whose load has not landed)."""
 import os
 import re
 import shutil
@@ -15,7 +15,7 @@ PKG = os.path.join(ROOT, "nano-vllm-spec-decode_amd")
 sys.path.insert(0, PKG)
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 
-from asm_paths import function_lines, unsafe_asm_loads  # noqa: E402
+from asm_paths import function_lines, unsafe_in_flight  # noqa: E402
 
 
 @pytest.fixture(scope="module")
@@ -32,11 +32,32 @@ def device_asm(tmp_path_factory):
     return open(out).read()
 
 
+def _kernels(asm):
+    return sorted(set(re.findall(r"^(_ZN2sd6lmhead9tile_gemm\w+):", asm, re.M)))
+
+
 def test_tile_gemm_loads_complete_before_use(device_asm):
-    symbols = sorted(set(re.findall(r"^(_ZN2sd6lmhead9tile_gemm\w+):", device_asm, re.M)))
-    assert len(symbols) == 10, symbols     # one per workgroup shape
+    symbols = _kernels(device_asm)
+    assert len(symbols) == 11, symbols     # one per workgroup shape
     for symbol in symbols:
-        bad, n = unsafe_asm_loads(function_lines(device_asm, symbol))
-        assert n >= 15 and not bad, (symbol, n, bad[:4])
+        bad, loads, reads = unsafe_in_flight(function_lines(device_asm, symbol))
+        tn, tm, da = (int(x) for x in re.search(r"TileILi(\d+)ELi(\d+)ELi\d+ELi\d+ELi(\d+)E", symbol).groups())
+        # the first DA - 1 steps' loads and one step's reads, then both for each of the DA steps of the loop
+        assert loads >= tn * (2 * da - 1) and reads >= tm * (da + 1), (symbol, loads, reads)
+        assert not bad, (symbol, bad[:4])
         scratch = re.search(r"; ScratchSize: (\d+)", device_asm[device_asm.index("\n" + symbol + ":"):])
         assert scratch and int(scratch.group(1)) == 0, symbol
+
+
+def test_check_finds_a_wait_too_short(device_asm):
+    """The check itself: each counted wait of a kernel's loop lengthened by one lets a load through."""
+    symbol = _kernels(device_asm)[0]
+    lines = function_lines(device_asm, symbol)
+    found = {"vmcnt": 0, "lgkmcnt": 0}
+    for i, (text, in_asm) in enumerate(lines):
+        m = re.match(r"s_waitcnt (vmcnt|lgkmcnt)\(([1-9]\d*)\)", text)
+        if in_asm and m:
+            planted = list(lines)
+            planted[i] = (f"s_waitcnt {m.group(1)}({int(m.group(2)) + 1})", True)
+            found[m.group(1)] += bool(unsafe_in_flight(planted)[0])
+    assert found["vmcnt"] and found["lgkmcnt"], found

@@ -48,7 +48,7 @@ def test_linear_vs_float64(device, M, N, K):
     _check_rows(x, w, y, list(range(0, M, max(1, M // 6))) + [M - 1])
 
 
-# 300 tiles: 256 whole ones and a split last round (the physical split at every row count, as the LM head)
+# 300 tiles: 256 of one range of k and 44 of five, unequal ones of S / 5 steps
 @pytest.mark.parametrize("name,K,N", QWEN3_8B + [("partly_split", 128, 76800)])
 def test_linear_rows_independent_of_row_count(device, name, K, N):
     g = torch.Generator(device=device).manual_seed(K + N)
@@ -136,6 +136,50 @@ def test_linear_kernel_edges(device, N, K):
         for i, r in enumerate(probes):
             if r < M:
                 assert torch.equal(y[r], alone[i]), f"row {r} of {M}"
+
+
+def _ranges(N, K):
+    """The layer's rule: packed tiles of 256 rows from `full` on are summed in n ranges of k (sd_linear's contract)."""
+    tiles = -(-N // 256)
+    tail = tiles - (tiles - 1) // 256 * 256
+    n = 1 if 2 * tail > 256 else min(8, 256 // tail, K // 64)
+    return (tiles, 1) if n < 2 else (tiles - tail, n)
+
+
+# How an output is summed, made visible: a weight row holds 2^28 in the first column, -2^28 in the last and quarters
+# between, in each range but the first for 4 m of its steps of 32 columns before the last. A range of its own keeps its
+# 32 m, and every sum on the way is exact (a multiple of 32 below 2^28 + 2^24); added to 2^28 step by step, the 8 of a
+# step are less than half a unit of 32 and all are lost. So outputs are 32 times the sum of m with the ranges and 0 in
+# a tile of one. Every kernel and workgroup shape, ranges that end anywhere in the steps ahead, rows of unlike signs.
+@pytest.mark.parametrize("N,K", [(1000, 1056), (4096, 4096), (4096, 12288), (6144, 1184), (24576, 4096), (76800, 1568),
+                                 (151936, 1024), (33000, 512)])
+def test_linear_sums_ranges_of_k(device, N, K):
+    full, n = _ranges(N, K)
+    S = K // 32
+    w = torch.zeros(K, dtype=torch.float64)
+    total = 0
+    for r in range(1, n):
+        begin, end = r * S // n, (r + 1) * S // n
+        m = (end - begin - 1) // 4
+        w[32 * begin:32 * (begin + 4 * m)] = 0.25
+        total += 32 * m
+    assert n == 1 or total > 0
+    w[0], w[K - 1] = 2.0 ** 28, -2.0 ** 28
+    single = torch.zeros(K, dtype=torch.float64)             # a tile of one range: quarters everywhere, all lost
+    single[0], single[32:K - 32], single[K - 1] = 2.0 ** 28, 0.25, -2.0 ** 28
+    scale = torch.tensor([1.0, -2.0, 4.0], dtype=torch.float64)[torch.arange(N) % 3]
+    cut = min(N, 256 * full)
+    weight = torch.empty(N, K, dtype=torch.bfloat16, device=device)
+    weight[:cut] = (scale[:cut, None].to(device) * single.to(device)).to(torch.bfloat16)
+    weight[cut:] = (scale[cut:, None].to(device) * w.to(device)).to(torch.bfloat16)
+    want = (scale * total * (torch.arange(N) >= cut)).to(torch.bfloat16).to(device)
+    lin = RowInvariantLinear(weight)
+    sign = (1.0 - 2.0 * (torch.arange(1168) % 2)).to(torch.bfloat16).to(device)
+    x = sign[:, None].expand(1168, K).contiguous()
+    for M in (1, 16, 17, 64, 80, 160, 320, 600, 1168) if N < 100000 else (5, 20, 64, 320):
+        print(f"M={M} N={N} K={K} ranges={n} from tile {full}", flush=True)
+        y = lin(x[:M])
+        assert torch.equal(y.float(), (sign[:M, None] * want).float()), f"M={M}"
 
 
 def test_linear_output_over_its_input(device):
