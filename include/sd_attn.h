@@ -115,10 +115,12 @@ int sd_paged_decode(const void* q, int64_t q_token_stride, const void* k_cache, 
  * K / V load policy of the planned calls: non-temporal when the contexts are balanced (longest at most twice
  * the mean), the default policy otherwise; sd_paged_decode always loads non-temporal. Order and policy only
  * decide which workgroup computes which sequence and how it loads: results are bitwise those of
- * sd_paged_decode even when the plan was made for other context lengths, as long as it was made for the
- * same num_seqs. With too few pairs to merge inside one workgroup and few rows a pair, the planned call's last
- * workgroup of a pair merges its partials (the plan clears the arrival counts in the workspace, each call leaves
- * them cleared).
+ * sd_paged_decode even when the plan was made for other context lengths, as long as it was made in this workspace for
+ * the same num_seqs, num_heads and num_kv_heads and for a num_query_tokens of as many 16-row tiles of query rows
+ * (num_query_tokens * num_heads / num_kv_heads rows); calls of at least 256 (sequence, KV head) pairs and at most 48
+ * query rows need the same num_seqs only. With fewer pairs and few rows the planned call's last workgroup of a pair
+ * merges its partials: the plan clears arrival counts in the workspace, each call leaves them cleared. Between a plan
+ * and its calls nothing may write the workspace but calls of these sizes, sd_paged_decode's included.
  * No counterpart in the reference; it serves the per-layer loop of a decode step
  * (nanovllm/engine/model_runner.py:476-485).
  */

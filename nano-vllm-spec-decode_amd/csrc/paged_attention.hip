@@ -1445,11 +1445,15 @@ struct Layout {
   size_t part_o, part_ml, work, count, work_pre, count_pre, order, arrivals, total;
 };
 
+// Arrival counts of merge_last: one a pair, and calls of more pairs do not use it (merges_last).
+constexpr int kArrivals = 256;
+
 // Workspace: residue partials only when a pair's residues span several workgroups (few items); for varlen, the
-// two work lists and their counts; for a planned decode call, the order and, with partials, the arrival counts of
-// the pairs (merge_last).
+// two work lists and their counts; for a planned decode call, the order and, with partials, kArrivals arrival counts.
+// Whether a call uses the counts depends on its query rows; where they are and that the plan clears them does not, so
+// that a plan serves every call whose order is at the same place.
 Layout workspace_layout(int64_t items, int Hkv, int rows_alloc, bool partials, bool varlen, int64_t pre_items = 0,
-                        int64_t order_len = 0, bool arrivals = false) {
+                        int64_t order_len = 0) {
   Layout L;
   const int64_t cells = partials ? items * Hkv * kResidues * rows_alloc : 0;
   L.part_o = 0;
@@ -1460,7 +1464,7 @@ Layout workspace_layout(int64_t items, int Hkv, int rows_alloc, bool partials, b
   L.count_pre = align256(L.work_pre + (varlen ? (size_t)pre_items * 2 * sizeof(int32_t) : 0));
   L.order = align256(L.count_pre + (varlen ? 2 * sizeof(int32_t) : 0));  // all q-blocks, those with keys
   L.arrivals = align256(L.order + (size_t)(order_len ? order_len + 1 : 0) * sizeof(int32_t));  // + load-policy flag
-  L.total = align256(L.arrivals + (arrivals ? (size_t)items * Hkv * sizeof(int32_t) : 0));
+  L.total = align256(L.arrivals + (order_len && partials ? kArrivals * sizeof(int32_t) : 0));
   return L;
 }
 
@@ -1499,10 +1503,10 @@ int residue_waves(int64_t items, int Hkv, int RT) {
 // rows over the GPU. Measured (us a layer, attn_combine -> merge_last, 8 KV heads): 4 rows, 1 x 300 keys 8.5 -> 8.0,
 // 1 x 4096 19.9 -> 19.3, 16 x 300 10.8 -> 10.4; 8 rows, 16 x 300 11.9 -> 10.9; between, 4 rows, 2 x 1000 10.1 ->
 // 10.8, 3 x 2000 the same, 8 x 300 9.1 -> 9.5; more than a pass: 20 rows, 1 x 4096 19.5 -> 20.5, 4 x 2000
-// 18.9 -> 21.8; 36 rows, 2 x 1000 11.5 -> 14.8.
+// 18.9 -> 21.8; 36 rows, 2 x 1000 11.5 -> 14.8. (Calls of at least kArrivals pairs have eight waves, or four row tiles.)
 bool merges_last(int waves, int64_t pairs, int merge_rows) {
   const int threads = waves == 1 ? kStreamThreads : waves * kWave;
-  return (waves == 4 || (waves == 1 && pairs <= 8)) && merge_rows * (kD / 4) <= threads;
+  return pairs <= kArrivals && (waves == 4 || (waves == 1 && pairs <= 8)) && merge_rows * (kD / 4) <= threads;
 }
 
 int check_heads(const char* who, int Hq, int Hkv, int D) {
@@ -1561,9 +1565,8 @@ extern "C" size_t sd_paged_decode_workspace_size(int32_t num_seqs, int32_t num_q
   int RT, P;
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
-  const int waves = residue_waves(items, num_kv_heads, RT);
-  const bool last = merges_last(waves, items * num_kv_heads, std::min(P * (num_heads / num_kv_heads), RT * 16));
-  return workspace_layout(items, num_kv_heads, RT * 16, waves < kResidues, false, 0, num_seqs, last).total;
+  const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
+  return workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs).total;
 }
 
 namespace {
@@ -1599,7 +1602,7 @@ int decode_run(const char* who, bool planned, const void* q, int64_t q_token_str
   const bool partials = waves < kResidues;
   const int merge_rows = std::min(P * g, RT * 16);  // rows a query group can hold, not the row tiles' padding
   const bool last = merges_last(waves, items * num_kv_heads, merge_rows);
-  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
+  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs);
   // The unplanned call needs the workspace only for partials; the planned one reads the order from it.
   const size_t need = planned ? lay.total : partials ? lay.order : 0;
   if (need && (!workspace || workspace_bytes < need))
@@ -1681,15 +1684,13 @@ extern "C" int sd_paged_decode_plan(const int32_t* context_lens, int32_t num_seq
   int RT, P;
   decode_shape(num_query_tokens, num_heads / num_kv_heads, &RT, &P);
   const int64_t items = (int64_t)num_seqs * ((num_query_tokens + P - 1) / P);
-  const int waves = residue_waves(items, num_kv_heads, RT);
-  const bool partials = waves < kResidues;
-  const bool last = merges_last(waves, items * num_kv_heads, std::min(P * (num_heads / num_kv_heads), RT * 16));
-  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs, last);
+  const bool partials = residue_waves(items, num_kv_heads, RT) < kResidues;
+  const Layout lay = workspace_layout(items, num_kv_heads, RT * 16, partials, false, 0, num_seqs);
   if (!workspace || workspace_bytes < lay.total)
     return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B", who, workspace_bytes, lay.total);
   hipLaunchKernelGGL(decode_plan, dim3(1), dim3(kPlanThreads), 0, (hipStream_t)stream, context_lens, num_seqs,
                      (int32_t*)((uint8_t*)workspace + lay.order), (int32_t*)((uint8_t*)workspace + lay.arrivals),
-                     last ? (int32_t)(items * num_kv_heads) : 0);
+                     partials ? kArrivals : 0);
   return check_launch(who);
 }
 

@@ -51,6 +51,10 @@ def test_workspace_sizes(lib):
     assert lib.sd_paged_decode_workspace_size(16, 9, 32, 8, 128, 256, 33) >= 16 * 8 * 8 * 48 * 130 * 4
     # 17 queries x 4 heads = 68 rows -> 4 row tiles (64 rows) in two query groups, never merged in LDS
     assert lib.sd_paged_decode_workspace_size(64, 17, 32, 8, 128, 256, 33) >= 128 * 8 * 8 * 64 * 130 * 4
+    # a workspace sized for a plan of more query tokens serves fewer (the arrival counts do not depend on the rows)
+    for seqs in (1, 2, 8, 16, 31):
+        sizes = [lib.sd_paged_decode_workspace_size(seqs, n, 32, 8, 128, 256, 33) for n in range(1, 17)]
+        assert sizes == sorted(sizes) and len(set(sizes[:4])) == 1, (seqs, sizes)
     assert lib.sd_paged_decode_workspace_size(0, 5, 32, 8, 128, 256, 33) == 0
     assert lib.sd_varlen_workspace_size(51, 2048, 4096, 32, 8, 128) > 0
     # per-row statistics of 6 spans (16 B each) for 64 x 5 target and 64 x 4 draft rows

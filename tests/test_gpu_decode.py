@@ -260,6 +260,36 @@ def test_planned_last_workgroup_merge_bitwise(device, B, n, Hq, Hkv):
         assert torch.equal(outs[i], refs[i]), i
 
 
+@pytest.mark.parametrize("B,plan_n,n", [(1, 4, 1), (1, 3, 2), (16, 3, 1), (16, 4, 2), (16, 1, 4), (1, 1, 3)])
+def test_plan_serves_other_query_counts(device, B, plan_n, n):
+    """C ABI: a plan made for plan_n query tokens serves planned calls of n in the same workspace (one row tile each),
+    whatever the workspace held before and whichever of the two merges in the last workgroup; a call between the two,
+    planned or not, changes nothing. Bitwise sd_paged_decode."""
+    from nanovllm_amd import _lib
+    lib, stream = _lib.load(), _lib.stream_of(device)
+    Hq, Hkv, bs = 32, 8, 256
+    rnd = random.Random(B + n)
+    ctx = [rnd.randint(5, 700) for _ in range(B)]
+    kc, vc, tables = paged_cache(device, ctx, Hkv, 128, seed=600)
+    lens = torch.tensor(ctx, dtype=torch.int32, device=device)
+    nbytes = max(lib.sd_paged_decode_workspace_size(B, m, Hq, Hkv, 128, bs, tables.size(1)) for m in (plan_n, n))
+    ws = torch.full((nbytes,), 0x55, dtype=torch.uint8, device=device)
+
+    def call(fn, m, q):
+        out = torch.full((B * m, Hq, 128), 7.0, dtype=torch.bfloat16, device=device)
+        _lib.check(fn(q.data_ptr(), q.stride(-3), kc.data_ptr(), vc.data_ptr(), kc.size(0), bs, lens.data_ptr(),
+                      tables.data_ptr(), tables.size(1), B, m, Hq, Hkv, 128, 128 ** -0.5, out.data_ptr(), out.stride(0),
+                      ws.data_ptr(), nbytes, stream), "decode")
+        return out
+
+    q = {m: queries(device, B * m, Hq, 128, seed=601 + m) for m in (plan_n, n)}
+    want = {m: paged_decode_attention(q[m].view(B, m, Hq, 128), kc, vc, lens, tables, 128 ** -0.5) for m in q}
+    _lib.check(lib.sd_paged_decode_plan(lens.data_ptr(), B, plan_n, Hq, Hkv, ws.data_ptr(), nbytes, stream), "plan")
+    for m, planned in [(n, True), (plan_n, True), (n, False), (n, True), (n, True)]:
+        out = call(lib.sd_paged_decode_planned if planned else lib.sd_paged_decode, m, q[m])
+        assert torch.equal(out.view_as(want[m]), want[m]), (m, planned)
+
+
 def test_planned_past_1024_sequences(device):
     """1100 sequences, more than the plan's 1024-thread sort (the dispatch order is then the index order, and
     the plan's scan takes two passes): the planned call equals the unplanned one bitwise, and a sample of
