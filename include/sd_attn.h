@@ -241,7 +241,8 @@ int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, int32_t hid
  * Each output row depends on its input row and the weight only, never on `rows`: the library GEMM picks kernels (and
  * summation orders) by the row count, which changes a model's greedy tokens with the batch; reference counterpart of
  * the property: scripts/check_padding.py:46-52 (GEMMs, padded vs alone). out may overlap x (the rows are then copied
- * to the workspace first). The workspace size is not monotonic in `rows`: size it for each row count a caller uses.
+ * to the workspace first, which must hold sd_linear_workspace_size bytes; a call whose out does not overlap x
+ * needs no workspace).
  */
 size_t sd_linear_workspace_size(int32_t rows, int32_t out_features, int32_t in_features);
 int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, const void* packed_weight, int32_t out_features,

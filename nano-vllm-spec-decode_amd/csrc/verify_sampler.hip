@@ -954,12 +954,14 @@ struct RowPlan {
 // less than the weight takes from HBM; of equal ones the first. A larger shape loads less per MFMA, a smaller one
 // keeps more CUs busy: at 320 rows 4096 x 4096 takes 25 us as 64 x 80 and 57 as 256 x 128, at 1168 rows
 // 24576 x 4096 207 us as 256 x 160 and 226 as 256 x 128. 256 x 256 has no registers for a sum of ranges: it takes
-// weights of one range a tile only (with its one-range sums 24576 x 4096 took 193 us).
-RowPlan row_plan(int M, int N, int K) {
+// weights of one range a tile only (with its one-range sums 24576 x 4096 took 193 us). max_tiles: shapes that cut the
+// weight into more tiles are left out (it is at least the packed tiles, which the 256-row shapes have).
+RowPlan row_plan(int M, int N, int K, int max_tiles = INT32_MAX) {
   if (M <= lmhead::kStreamRows) {
-    if (N >= 512 * lmhead::kN) return {k256x32, (N + lmhead::kN - 1) / lmhead::kN, 1};
     const bool wide = N >= 192 * 32;
-    return {wide ? kStream32 : kStream16, (N + (wide ? 31 : 15)) / (wide ? 32 : 16), 1};
+    const int stream_tiles = (N + (wide ? 31 : 15)) / (wide ? 32 : 16);
+    if (N >= 512 * lmhead::kN || stream_tiles > max_tiles) return {k256x32, (N + lmhead::kN - 1) / lmhead::kN, 1};
+    return {wide ? kStream32 : kStream16, stream_tiles, 1};
   }
   struct Shape {
     RowShape shape;
@@ -979,6 +981,7 @@ RowPlan row_plan(int M, int N, int K) {
     // the ranges' ends are multiples of `ends` if the ranges are equal and multiples themselves
     if (splits > 1 && (c.ends == 0 || (c.ends > 1 && steps % (splits * c.ends)))) continue;
     const int tn = (N + c.rows_n - 1) / c.rows_n, tm = (M + c.rows_m - 1) / c.rows_m;
+    if (tn > max_tiles) continue;
     const int64_t rounds = ((int64_t)tn * tm + kCUs - 1) / kCUs;
     const int64_t ns = std::max(hbm_ns, rounds * ((int64_t)steps * c.step_ns + kStartNs));
     if (ns < best_ns) {
@@ -995,8 +998,7 @@ void launch_tile(const lmhead::Args& a, hipStream_t s) {
   hipLaunchKernelGGL(lmhead::tile_gemm<T>, dim3(grid), dim3(T::kThreads), 0, s, a);
 }
 
-int launch_row_gemm(lmhead::Args a, hipStream_t s) {
-  const RowPlan p = row_plan(a.M, a.N, a.K);
+int launch_row_gemm(lmhead::Args a, const RowPlan& p, hipStream_t s) {
   const lmhead::Ranges ranges = lmhead::sum_ranges(a.N, a.K);
   a.tiles_n = p.tiles_n;
   a.tiles_m = p.tiles_m;
@@ -1040,57 +1042,31 @@ int copy_input(lmhead::Args* a, uint16_t* dst, hipStream_t s) {
   return check_launch("copy_rows");
 }
 
-// Workspace sizes of sd_linear and sd_lm_head_verify. They are part of the C ABI (a caller may hold a size it asked
-// for earlier, and a smaller workspace is refused), so the reported size stays that of a reduction split along k
-// into fp32 range sums: the packed rows (a multiple of 64 MB rows, MB the 32-row blocks of a 2-wave column of at
-// most 320 rows) and, per row of workgroups, the sums of the split tiles. The kernels above need no more than a copy
-// of the rows, and for the LM head the argmax candidates.
-constexpr int kAbiCUs = 256, kAbiMaxRows = 320;
-int abi_mb(int64_t M) { return (int)std::min<int64_t>(5, std::max<int64_t>(1, ((M + 31) / 32 + 1) / 2)); }
-struct AbiSplit {
-  int64_t tail;
-  int splits;
-};
-AbiSplit abi_split(int N, int K) {
-  const int tiles = (N + lmhead::kN - 1) / lmhead::kN;
-  const int tail = tiles - (tiles - 1) / kAbiCUs * kAbiCUs;
-  const int splits = 2 * tail > kAbiCUs ? 1 : std::min({8, kAbiCUs / tail, K / (2 * lmhead::kK)});
-  return {splits < 2 ? 0 : tail, std::max(splits, 1)};
-}
-size_t abi_sums(int64_t grid_rows, int MB, const AbiSplit& sp) {
-  return (size_t)(grid_rows * sp.tail * sp.splits) * 8 * 2 * MB * 16 * kWave * sizeof(float);
-}
+// Workspace of sd_linear: a copy of the token rows, which only a call whose output overlaps them makes.
+size_t linear_workspace(int M, int K) { return align256((size_t)M * K * 2); }
 
-size_t linear_workspace(int M, int N, int K) {
-  const int tiles = (N + lmhead::kN - 1) / lmhead::kN;
-  const AbiSplit sp = abi_split(N, K);
-  const int MB = abi_mb(M);
-  const bool in_order = M > kAbiMaxRows && sp.splits > 1 && sp.tail == tiles;   // its range sums stayed in registers
-  const int64_t unit = in_order ? 128 : 64 * MB;
-  const int64_t mpad = ((int64_t)M + unit - 1) / unit * unit;
-  return align256(align256((size_t)mpad * K * 2) + (in_order ? 0 : abi_sums(mpad / (64 * MB), MB, sp)));
-}
-
+// Workspace of the LM head: the statistics and decisions of its rows, then the argmax candidates, one a row and tile of
+// the call's shape; in a call whose logits overlap its rows, those of a 256-row shape and the rows' copy.
 struct LmLayout {
-  size_t best, stats, info, copy, total;
+  size_t stats, info, best, copy, total;
+  int max_tiles, overlap_tiles;   // candidates a row has room for, and in a call with the copy
 };
 LmLayout lm_layout(int S, int K, int V, int H) {
   const int64_t M = (int64_t)S * (K + 1);
-  const int tiles = (V + lmhead::kN - 1) / lmhead::kN;
-  LmLayout L;
-  L.best = 0;
   const int rows = (int)std::min<int64_t>(M, INT32_MAX);
-  L.stats = align256((size_t)M * row_plan(rows, V, H).tiles_n * sizeof(lmhead::TileBest));
-  L.info = align256(L.stats + (size_t)M * sizeof(RowStat));
-  L.copy = align256(L.info + (size_t)S * sizeof(SeqInfo));
-  const int MB = abi_mb(M);
-  const int64_t mpad = (M + 64 * MB - 1) / (64 * MB) * (64 * MB);
-  size_t abi = align256((size_t)M * tiles * sizeof(lmhead::TileBest));
-  abi = align256(abi + (size_t)M * sizeof(RowStat));
-  abi = align256(abi + (size_t)S * sizeof(SeqInfo));
-  abi = align256(abi + (size_t)mpad * H * 2);
-  abi = align256(abi + abi_sums(mpad / (64 * MB), MB, abi_split(V, H)));
-  L.total = std::max(align256(L.copy + (size_t)M * H * 2), abi);
+  LmLayout L;
+  L.overlap_tiles = (V + lmhead::kN - 1) / lmhead::kN;
+  // Never more than a caller may have been told for these sizes when the workspace held the candidates of 256-row tiles
+  // and the rows, packed and padded to 64: shapes of more tiles are left out where they would take more (calls of few
+  // hidden columns or a very wide vocabulary).
+  const int64_t packed = (M + 63) / 64 * 64 * H * 2;
+  L.max_tiles = (int)std::min<int64_t>(L.overlap_tiles + packed / (M * (int64_t)sizeof(lmhead::TileBest)), INT32_MAX);
+  L.stats = 0;
+  L.info = align256((size_t)M * sizeof(RowStat));
+  L.best = align256(L.info + (size_t)S * sizeof(SeqInfo));
+  L.copy = align256(L.best + (size_t)M * L.overlap_tiles * sizeof(lmhead::TileBest));
+  const size_t best = (size_t)M * row_plan(rows, V, H, L.max_tiles).tiles_n * sizeof(lmhead::TileBest);
+  L.total = std::max(align256(L.best + best), align256(L.copy + (size_t)M * H * 2));
   return L;
 }
 
@@ -1267,11 +1243,12 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
   a.out_vec = (uintptr_t)logits_out % 16 == 0 && logits_out_row_stride % 8 == 0;
   a.out_nt = 1;  // 64 rows with their logits 237.7 -> 221.6 us, 80 rows 244.7 -> 229.0
   a.best = temperatures ? nullptr : (lmhead::TileBest*)((uint8_t*)workspace + lay.best);
+  const bool overlap =
+      logits_out && rows_overlap(hidden, hidden_rows, hidden_row_stride, H, logits_out, M, logits_out_row_stride, V);
+  const RowPlan plan = row_plan(a.M, V, H, !a.best ? INT32_MAX : overlap ? lay.overlap_tiles : lay.max_tiles);
   int rc;
-  if (logits_out && rows_overlap(hidden, hidden_rows, hidden_row_stride, H, logits_out, M, logits_out_row_stride, V) &&
-      (rc = copy_input(&a, (uint16_t*)((uint8_t*)workspace + lay.copy), s)))
-    return rc;
-  if ((rc = launch_row_gemm(a, s))) return rc;
+  if (overlap && (rc = copy_input(&a, (uint16_t*)((uint8_t*)workspace + lay.copy), s))) return rc;
+  if ((rc = launch_row_gemm(a, plan, s))) return rc;
   auto poison = [&]() -> int {
     if (!logits_indices) return kOk;
     hipLaunchKernelGGL(lm_head_poison, dim3((unsigned)((S + 63) / 64)), dim3(64), 0, s, logits_indices, hidden_rows, S,
@@ -1298,8 +1275,7 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
   p.out_next = next_token;
   p.stats = (RowStat*)((uint8_t*)workspace + lay.stats);
   p.info = (SeqInfo*)((uint8_t*)workspace + lay.info);
-  hipLaunchKernelGGL(lm_head_merge, dim3((unsigned)M), dim3(kThreads), 0, s, a.best, row_plan(a.M, V, H).tiles_n,
-                     p.stats);
+  hipLaunchKernelGGL(lm_head_merge, dim3((unsigned)M), dim3(kThreads), 0, s, a.best, plan.tiles_n, p.stats);
   if ((rc = check_launch("lm_head_merge"))) return rc;
   hipLaunchKernelGGL((verify_decide<SD_DTYPE_BF16, SD_DTYPE_BF16, false>), dim3(S), dim3(64), 0, s, p);
   if ((rc = check_launch("verify_decide"))) return rc;
@@ -1308,7 +1284,7 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
 
 extern "C" size_t sd_linear_workspace_size(int32_t rows, int32_t out_features, int32_t in_features) {
   if (rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % lmhead::kK) return 0;
-  return linear_workspace(rows, out_features, in_features);
+  return linear_workspace(rows, in_features);
 }
 
 extern "C" int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, const void* packed_weight,
@@ -1325,9 +1301,10 @@ extern "C" int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, cons
     return fail(kBadArgument, "%s: a row stride is smaller than the row", who);
   if (((uintptr_t)x | (uintptr_t)packed_weight) % 16 || x_row_stride % 8 || (uintptr_t)out % 2)
     return fail(kUnsupported, "%s: x needs 16-byte aligned rows (row stride a multiple of 8 elements)", who);
-  const size_t need = linear_workspace(M, N, K);
-  if (!workspace || workspace_bytes < need)
-    return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B", who, workspace_bytes, need);
+  const bool overlap = rows_overlap(x, M, x_row_stride, K, out, M, out_row_stride, N);
+  const size_t need = overlap ? linear_workspace(M, K) : 0;
+  if (need && (!workspace || workspace_bytes < need))
+    return fail(kWorkspaceTooSmall, "%s: workspace %zu B < %zu B (out overlaps x)", who, workspace_bytes, need);
   hipStream_t s = (hipStream_t)stream;
   lmhead::Args a{};
   a.x = (const uint16_t*)x;
@@ -1341,7 +1318,6 @@ extern "C" int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, cons
   a.out_stride = out_row_stride;
   a.out_vec = (uintptr_t)out % 16 == 0 && out_row_stride % 8 == 0;
   int rc;
-  if (rows_overlap(x, M, x_row_stride, K, out, M, out_row_stride, N) && (rc = copy_input(&a, (uint16_t*)workspace, s)))
-    return rc;
-  return launch_row_gemm(a, s);
+  if (overlap && (rc = copy_input(&a, (uint16_t*)workspace, s))) return rc;
+  return launch_row_gemm(a, row_plan(M, N, K), s);
 }

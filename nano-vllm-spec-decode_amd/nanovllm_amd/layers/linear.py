@@ -27,15 +27,18 @@ class RowInvariantLinear:
         if x.dtype != torch.bfloat16 or x.dim() != 2 or x.size(1) != self.in_features or x.stride(1) != 1:
             raise ValueError("RowInvariantLinear: bf16 [rows, in_features] with unit column stride required")
         M = x.size(0)
-        if out is None:
+        fresh = out is None
+        if fresh:
             out = torch.empty(M, self.out_features, dtype=torch.bfloat16, device=x.device)
         if out.dtype != torch.bfloat16 or out.shape != (M, self.out_features) or out.stride(1) != 1:
             raise ValueError("RowInvariantLinear: out must be bf16 [rows, out_features] with unit column stride")
         if M == 0:
             return out
         lib = _lib.load()
-        ws = _lib.workspace(lib.sd_linear_workspace_size(M, self.out_features, self.in_features), x.device)
+        # a given out may overlap x: the rows' copy goes to the workspace then
+        nbytes = 0 if fresh else lib.sd_linear_workspace_size(M, self.out_features, self.in_features)
+        ws = _lib.workspace(nbytes, x.device) if nbytes else None
         _lib.check(lib.sd_linear(x.data_ptr(), x.stride(0), M, self.packed.data_ptr(), self.out_features,
-                                 self.in_features, out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(),
-                                 _lib.stream_of(x.device)), "sd_linear")
+                                 self.in_features, out.data_ptr(), out.stride(0), _lib.ptr(ws),
+                                 ws.numel() if ws is not None else 0, _lib.stream_of(x.device)), "sd_linear")
         return out

@@ -59,13 +59,29 @@ def test_workspace_sizes(lib):
     assert lib.sd_varlen_workspace_size(51, 2048, 4096, 32, 8, 128) > 0
     # per-row statistics of 6 spans (16 B each) for 64 x 5 target and 64 x 4 draft rows
     assert lib.sd_verify_workspace_size(64, 4, 151936, 1) >= (64 * 5 + 64 * 4) * 6 * 16
-    # sd_linear, qkv shape (24 tiles, each split into 8 ranges): up to 320 rows the packed rows plus every
-    # range's fp32 sums (one row of workgroups: 24 x 8 x 327,680 B); past it the ranges run in order in one
-    # workgroup, so only the packed rows (1168 -> 1280 rows of 4096 bf16); not monotonic in the rows
-    small, large = lib.sd_linear_workspace_size(320, 6144, 4096), lib.sd_linear_workspace_size(1168, 6144, 4096)
-    assert small >= 320 * 4096 * 2 + 24 * 8 * 327680 and large == 1280 * 4096 * 2 and large < small
-    # a vocabulary-sized projection keeps the physical split at any row count: sums for every row of workgroups
-    assert lib.sd_linear_workspace_size(640, 151936, 4096) >= 640 * 4096 * 2 + 2 * 82 * 3 * 327680
+    # sd_linear: a copy of the rows (for an out over x), whatever the weight's rows; never more than the packed rows
+    # and fp32 range sums that these calls asked for when the ranges were workgroups of their own
+    for rows, n, k, before in [(320, 6144, 4096, 320 * 4096 * 2 + 24 * 8 * 327680), (1168, 6144, 4096, 1280 * 4096 * 2),
+                               (640, 151936, 4096, 640 * 4096 * 2 + 2 * 82 * 3 * 327680)]:
+        assert lib.sd_linear_workspace_size(rows, n, k) == rows * k * 2 < before
+
+
+def test_lm_head_workspace_never_grew(lib):
+    """The LM head's workspace against what the same call asked for when it held the argmax candidates of 256-row
+    tiles, row statistics (16 B), decisions (48 B), the packed rows (padded to 64) and, where the last round of tiles was split,
+    range sums (left out here): a caller's buffer of then is still enough, and little is asked for at Qwen3-8B."""
+    al = lambda b: -(-b // 256) * 256  # noqa: E731
+    for seqs, k, vocab, hidden in [(64, 0, 128256, 4096), (16, 4, 128256, 2048), (16, 0, 128256, 512), (16, 0, 131000, 32),
+                                   (4, 3, 65536, 128), (64, 4, 151936, 4096), (1, 0, 32000, 64), (200, 4, 128256, 64),
+                                   (7, 2, 50257, 32), (33, 0, 200000, 1024)]:
+        rows, tiles = seqs * (k + 1), -(-vocab // 256)
+        mb = min(5, max(1, ((rows + 31) // 32 + 1) // 2))
+        packed = -(-rows // (64 * mb)) * 64 * mb * hidden * 2
+        info = lib.sd_lm_head_verify_workspace_size(seqs, k, vocab, hidden, 0)
+        verify = lib.sd_verify_workspace_size(seqs, k, vocab, 0)
+        assert info <= max(verify, al(rows * tiles * 8) + al(rows * 16) + al(seqs * 48) + al(packed)), (
+            seqs, k, vocab, hidden, info)
+    assert lib.sd_lm_head_verify_workspace_size(64, 4, 151936, 4096, 0) < 8 << 20
 
 
 def test_bad_arguments_return_status(lib):
@@ -112,8 +128,7 @@ def test_bad_arguments_return_status(lib):
     rc = lib.sd_linear(None, 4096, 4, None, 6144, 4096, None, 6144, None, 0, None)
     assert rc == 1 and b"null pointer" in lib.sd_last_error()
     assert lib.sd_linear(None, 0, 0, None, 6144, 4096, None, 0, None, 0, None) == 0            # nothing to do
-    # packed rows [Mpad=64][4096] bf16, then [1 row of workgroups][16 split tiles][8 ranges] of fp32 sums
-    assert lib.sd_linear_workspace_size(1, 4096, 4096) == 64 * 4096 * 2 + 16 * 8 * 8 * 2 * 1 * 16 * 64 * 4
+    assert lib.sd_linear_workspace_size(1, 4096, 4096) == 4096 * 2
     rn = lib.sd_rms_norm
     rc = rn(None, 4096, None, 0, None, 1e-6, 4, 4100, None, 4096, None, 0, None)
     assert rc == 2 and b"multiple of 8" in lib.sd_last_error()

@@ -209,3 +209,36 @@ def test_lm_head_bad_logits_index_marks_its_sequence(device):
                 assert a[s] == -1 and t[s] == -1
             else:
                 assert a[s] == a_ok[s] and t[s] == t_ok[s]
+
+
+@pytest.mark.parametrize("S,K,V,H,over", [(3, 2, 5000, 256, False), (16, 0, 20000, 64, False), (64, 4, 9000, 512, False),
+                                          (20, 0, 40000, 96, False), (64, 0, 70000, 64, False), (3, 2, 5000, 256, True),
+                                          (16, 0, 20000, 64, True), (64, 4, 9000, 512, True), (64, 0, 70000, 64, True)])
+def test_lm_head_workspace_and_logits_over_hidden(device, monkeypatch, S, K, V, H, over):
+    """Greedy calls in a workspace of exactly the size asked for (few hidden columns leave out shapes of many tiles),
+    with the logits in a buffer of their own or over the hidden rows (copied first): nothing past the workspace is
+    written, tokens are the oracle's on the logits, and the logits do not depend on where they go."""
+    from nanovllm_amd import _lib
+    M = S * (K + 1)
+    hidden, weight, _ = _inputs(device, 31, S, K, V, H)
+    head = LMHeadVerifier(weight)
+    drafts = torch.randint(0, V, (S, K), generator=torch.Generator().manual_seed(3)).to(device)
+    nd = torch.full((S,), K, dtype=torch.int64, device=device)
+    zeros = torch.zeros(S, device=device)
+    want = torch.empty(M, V, dtype=torch.bfloat16, device=device)
+    lm_head_verify(hidden, head, drafts, nd, zeros, logits_out=want)
+    _check_logits(hidden, weight, None, want, [0, M // 2, M - 1])
+    buf = torch.full((_lib.load().sd_lm_head_verify_workspace_size(S, K, V, H, 0) + 4096,), 0x5a, dtype=torch.uint8,
+                     device=device)
+    asked = []
+    monkeypatch.setattr(_lib, "workspace", lambda n, dev, tag="": asked.append(n) or buf[:n])
+    out = torch.empty(M, V, dtype=torch.bfloat16, device=device)
+    x = hidden
+    if over:
+        x = out.view(-1)[:M * H].view(M, H)
+        x.copy_(hidden)
+    acc, nxt = lm_head_verify(x, head, drafts, nd, zeros, logits_out=out)
+    assert torch.equal(out, want)
+    assert bool((buf[asked[0]:] == 0x5a).all())
+    ref_acc, ref_nxt = osmp.verify_drafts(want.cpu(), drafts.cpu(), nd.cpu(), zeros.cpu())
+    assert torch.equal(acc.cpu(), ref_acc) and torch.equal(nxt.cpu(), ref_nxt)
