@@ -61,7 +61,7 @@ struct Args {
   int32_t N, K;
   uint16_t* out;            // null, or [M, N] bf16 with row stride out_stride
   int64_t out_stride;
-  int32_t out_vec;          // out rows 16-byte aligned: 8 entries per store
+  int32_t out_align;        // what out and its row stride are multiples of: 16, 8 or 2 bytes (8, 4 or 1 entries a store)
   int32_t out_nt;           // non-temporal stores of whole lines (logits: they leave the token rows in L2)
   TileBest* best;           // [M][tiles_n], or null (no argmax)
   int32_t tiles_n, tiles_m;
@@ -317,7 +317,7 @@ __global__ __launch_bounds__(kWave) void stream_gemm(Args a) {
     const uint2 w = round4(a, sum[i] + acc[i], valid, n, bv, bi);
     if (!a.out || r16 >= a.M) continue;
     uint16_t* dst = a.out + (int64_t)r16 * a.out_stride + n;
-    if (n + 3 < a.N && a.out_vec) {
+    if (n + 3 < a.N && a.out_align >= 8) {
       *(uint2*)dst = w;
     } else {
       const uint16_t bits[4] = {(uint16_t)w.x, (uint16_t)(w.x >> 16), (uint16_t)w.y, (uint16_t)(w.y >> 16)};
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(T::kThreads, 1) void tile_gemm(Args a) {
   const int rows = min(MT, a.M - m0), cols = min(NT, a.N - nt * NT);
   if (a.out) {
     uint16_t* out = a.out + (int64_t)m0 * a.out_stride + nt * NT;
-    if (a.out_vec && cols == NT) {
+    if (a.out_align == 16 && cols == NT) {
       auto store_rows = [&](auto ntc) __attribute__((always_inline)) {
         for (int idx = threadIdx.x; idx < rows * kChunks; idx += T::kThreads) {
           const int mr = idx / kChunks, c = idx % kChunks;
@@ -561,6 +561,20 @@ __global__ __launch_bounds__(T::kThreads, 1) void tile_gemm(Args a) {
         store_rows(std::true_type{});
       else
         store_rows(std::false_type{});
+    } else if (a.out_align >= 8) {   // and the last columns of a ragged weight
+      for (int idx = threadIdx.x; idx < rows * (NT / 4); idx += T::kThreads) {
+        const int mr = idx / (NT / 4), n = 4 * (idx % (NT / 4));
+        const uint2 w = *(const uint2*)(lds + mr * (2 * NT) + (((n / 8) ^ (mr & kSwz)) << 4) + 2 * (n % 8));
+        uint16_t* dst = out + mr * a.out_stride + n;
+        if (n + 3 < cols) {
+          *(uint2*)dst = w;
+        } else {
+          const uint16_t bits[4] = {(uint16_t)w.x, (uint16_t)(w.x >> 16), (uint16_t)w.y, (uint16_t)(w.y >> 16)};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < cols) dst[e] = bits[e];
+        }
+      }
     } else {
       for (int idx = threadIdx.x; idx < rows * NT; idx += T::kThreads) {
         const int mr = idx / NT, n = idx % NT;

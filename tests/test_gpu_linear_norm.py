@@ -138,6 +138,24 @@ def test_linear_kernel_edges(device, N, K):
                 assert torch.equal(y[r], alone[i]), f"row {r} of {M}"
 
 
+# The same bits wherever the output's rows start: multiples of 16, 8 and 2 bytes (a store of 8, 4 and 1 entries), at
+# every kernel, a weight that ends inside a store and nothing written beside the rows.
+@pytest.mark.parametrize("N,K", [(1003, 96), (4094, 544), (24577, 64), (6144, 256)])
+def test_linear_output_alignment(device, N, K):
+    g = torch.Generator(device=device).manual_seed(N)
+    x = torch.randn(600, K, device=device, generator=g).to(torch.bfloat16)
+    lin = RowInvariantLinear((torch.randn(N, K, device=device, generator=g) * K ** -0.5).to(torch.bfloat16))
+    width = -(-(N + 16) // 8) * 8
+    for M in (3, 16, 40, 80, 160, 300, 600):
+        want = lin(x[:M])
+        for at, row in ((8, width), (4, width), (8, width + 4), (4, width + 4), (2, width), (3, width + 1)):
+            print(f"M={M} N={N} K={K} offset {at} row {row}", flush=True)
+            buf = torch.full((M, row), 7.0, dtype=torch.bfloat16, device=device)
+            lin(x[:M], out=buf[:, at:at + N])
+            assert torch.equal(buf[:, at:at + N], want)
+            assert bool((buf[:, :at] == 7).all()) and bool((buf[:, at + N:] == 7).all())
+
+
 def _ranges(N, K):
     """The layer's rule: packed tiles of 256 rows from `full` on are summed in n ranges of k (sd_linear's contract)."""
     tiles = -(-N // 256)
