@@ -1028,12 +1028,16 @@ int row_align(const void* x, int64_t stride) {
   return bits % 16 == 0 ? 16 : bits % 8 == 0 ? 8 : 2;
 }
 
-// Whether the byte ranges of two row tables overlap.
+// Whether two row tables share memory: their byte ranges overlap, and they are not column slices of one buffer side by
+// side (one row stride, y's columns past x's and before x's next row).
 bool rows_overlap(const void* x, int64_t x_rows, int64_t x_stride, int64_t x_cols, const void* y, int64_t y_rows,
                   int64_t y_stride, int64_t y_cols) {
   const uintptr_t x0 = (uintptr_t)x, y0 = (uintptr_t)y;
   const uintptr_t x1 = x0 + 2 * ((x_rows - 1) * x_stride + x_cols), y1 = y0 + 2 * ((y_rows - 1) * y_stride + y_cols);
-  return x0 < y1 && y0 < x1;
+  if (!(x0 < y1 && y0 < x1)) return false;
+  if (x_stride != y_stride) return true;
+  const int64_t stride = 2 * x_stride, diff = (int64_t)(y0 - x0), at = (diff % stride + stride) % stride;
+  return at < 2 * x_cols || at + 2 * y_cols > stride;
 }
 
 // A call whose output overlaps its input reads a copy of its token rows (in `dst`, M x K) instead.

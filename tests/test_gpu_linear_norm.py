@@ -156,6 +156,27 @@ def test_linear_output_alignment(device, N, K):
             assert bool((buf[:, :at] == 7).all()) and bool((buf[:, at + N:] == 7).all())
 
 
+# x and out in one buffer: a row copy (the workspace) only where they share memory. [x | out] and [out | x] side by side
+# don't, also with other rows between (x from row 2 on); one shared column, or out running into x's next row, does.
+@pytest.mark.parametrize("M", [3, 100])
+@pytest.mark.parametrize("xat,oat,row,shift,copied", [(0, 96, 352, 0, False), (256, 0, 352, 0, False), (0, 96, 352, 2, False),
+                                                      (256, 0, 352, 2, False), (0, 88, 352, 0, True), (256, 8, 352, 0, True),
+                                                      (0, 96, 344, 2, True), (0, 0, 352, 0, True)])
+def test_linear_column_slices_of_one_buffer(device, monkeypatch, M, xat, oat, row, shift, copied):
+    from nanovllm_amd import _lib
+    g = torch.Generator(device=device).manual_seed(M + xat)
+    lin = RowInvariantLinear((torch.randn(256, 96, device=device, generator=g) / 10).to(torch.bfloat16))
+    flat = torch.zeros((M + shift + 1) * row + 512, dtype=torch.bfloat16, device=device)
+    x = flat.as_strided((M, 96), (row, 1), shift * row + xat)
+    out = flat.as_strided((M, 256), (row, 1), oat)
+    x.copy_(torch.randn(M, 96, device=device, generator=g).to(torch.bfloat16))
+    want = lin(x)
+    ws = torch.full((1 << 16,), 0x5a, dtype=torch.uint8, device=device)
+    monkeypatch.setattr(_lib, "workspace", lambda n, dev, tag="": ws)
+    assert torch.equal(lin(x, out=out), want)
+    assert bool((ws != 0x5a).any()) == copied
+
+
 def _ranges(N, K):
     """The layer's rule: packed tiles of 256 rows from `full` on are summed in n ranges of k (sd_linear's contract)."""
     tiles = -(-N // 256)
