@@ -12,6 +12,8 @@ def silu_and_mul(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tens
     M, half = x.shape[0], x.shape[1] // 2
     if out is None:
         out = torch.empty(M, half, dtype=x.dtype, device=x.device)
+    if out.dtype != x.dtype or out.shape != (M, half) or out.stride(1) != 1 or out.device != x.device:
+        raise ValueError("silu_and_mul: out must be bf16 [rows, columns] with unit column stride on x's device")
     _lib.check(_lib.load().sd_silu_mul(x.data_ptr(), x.stride(0), M, half, out.data_ptr(), out.stride(0),
                                        _lib.stream_of(x.device)), "sd_silu_mul")
     return out
