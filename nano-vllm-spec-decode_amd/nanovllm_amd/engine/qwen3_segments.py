@@ -16,10 +16,11 @@ The norms follow the reference's RMSNorm arithmetic (nanovllm/layers/layernorm.p
 rsqrt, cast, times the weight); the GEMMs are torch's (hipBLASLt).
 
 row_invariant=True runs the projections through RowInvariantLinear (sd_linear), the norms through sd_rms_norm
-(which update the residual in place) and the activation through sd_silu_mul instead: every op then computes a token's row the same way whatever the step's token count, so a
-token's hidden state, and the greedy token picked from it, do not depend on the batch. That is what makes
-greedy speculative decoding (1 + k rows per sequence) pick exactly the tokens of plain decoding (one row); with
-the library GEMMs and reductions, whose kernels change with the row count, near-ties can flip.
+(which update the residual in place, except in the last segment) and the activation through sd_silu_mul instead:
+every op then computes a token's row the same way whatever the step's token count, so a token's hidden state, and
+the greedy token picked from it, do not depend on the batch. That is what makes greedy speculative decoding (1 + k
+rows per sequence) pick exactly the tokens of plain decoding (one row); with the library GEMMs and reductions, whose
+kernels change with the row count, near-ties can flip.
 """
 from __future__ import annotations
 
@@ -99,18 +100,18 @@ class Qwen3Segments:
         return torch.mm(x, w[name].t(), out=out)
 
     def _norm(self, x: torch.Tensor, weight: torch.Tensor, residual: torch.Tensor | None = None,
-              out: torch.Tensor | None = None):
-        if self.row_invariant:   # the residual is updated in place
-            return layernorm.rms_norm(x, weight, self.eps, residual, out=out, residual_out=residual)
+              out: torch.Tensor | None = None, in_place: bool = True):
+        if self.row_invariant:   # in_place: the residual is updated where it is
+            return layernorm.rms_norm(x, weight, self.eps, residual, out=out, residual_out=residual if in_place else None)
         res = rms_norm(x, weight, self.eps) if residual is None else add_rms_norm(x, residual, weight, self.eps)
         if out is not None:
             out.copy_(res if residual is None else res[0])
         return res
 
-    def _post_attn(self, w: dict, o: torch.Tensor, residual: torch.Tensor):
+    def _post_attn(self, w: dict, o: torch.Tensor, residual: torch.Tensor, in_place: bool):
         """Qwen3DecoderLayer.post_attn (qwen3.py:192-201)."""
         h = self._linear(o, w, "o")
-        h, residual = self._norm(h, w["post_norm"], residual)
+        h, residual = self._norm(h, w["post_norm"], residual, in_place=in_place)
         h = self._linear(h, w, "gate_up")
         if self.row_invariant:
             return self._linear(silu_and_mul(h), w, "down"), residual
@@ -122,7 +123,8 @@ class Qwen3Segments:
             h = F.embedding(self.input_ids[:n], self.embed)
             x, residual = self._norm(h, self.layers[0]["in_norm"]), h
         else:
-            h, residual = self._post_attn(self.layers[i - 1], bufs["o"][:n].view(n, -1), self.residual[:n])
+            # the last segment leaves the residual as it found it: it may run again on the same buffers
+            h, residual = self._post_attn(self.layers[i - 1], bufs["o"][:n].view(n, -1), self.residual[:n], i < self.L)
             if i == self.L:
                 self._norm(h, self.final_norm, residual, out=self.hidden_out[:n])
                 return

@@ -167,3 +167,20 @@ def test_model_greedy_spec_equals_plain(device):
     for L, a, b in zip(lens, plain, [s.token_ids for s in seqs]):
         n = L + steps + 1
         assert a[:n] == b[:n], f"spec tokens differ from plain tokens: {a[L:n]} vs {b[L:n]}"
+
+
+@pytest.mark.parametrize("row_invariant", [False, True])
+def test_last_segment_runs_again_on_the_same_buffers(device, row_invariant):
+    """The last segment reads the residual and the attention output and writes hidden_out only: a second run on the
+    same buffers (a retry, another head) gives the same hidden states."""
+    model = Qwen3Segments(num_layers=2, hidden=256, num_heads=4, num_kv_heads=2, head_dim=128, intermediate=512,
+                          vocab=1000, max_tokens=32, device=device, row_invariant=row_invariant)
+    n = 20
+    bufs = dict(o=torch.randn(32, 4, 128, device=device).to(torch.bfloat16),
+                qkv=torch.zeros(32, 8 * 128, dtype=torch.bfloat16, device=device))
+    model.input_ids.copy_(torch.arange(32) * 7 % 1000)
+    for i in range(3):
+        model(i, n, bufs)
+    first, residual = model.hidden_out.clone(), model.residual.clone()
+    model(2, n, bufs)
+    assert torch.equal(model.hidden_out, first) and torch.equal(model.residual, residual)
