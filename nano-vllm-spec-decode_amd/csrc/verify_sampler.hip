@@ -941,7 +941,7 @@ __global__ __launch_bounds__(64) void lm_head_poison(const int64_t* rows, int32_
 
 // The kernel a row-invariant GEMM call runs: every choice gives the same bits, so the rule looks at time alone.
 enum RowShape { kStream16, kStream32, k256x32, k32x64E16, k32x64, k32x80, k64x80, k128x64, k128x80, k128x160, k256x128,
-                k256x160, k256x256 };
+                k256x160, k256x256, kRowShapes };
 struct RowPlan {
   RowShape shape;
   int tiles_n, tiles_m;
@@ -1018,6 +1018,7 @@ int launch_row_gemm(lmhead::Args a, const RowPlan& p, hipStream_t s) {
     case k256x128: launch_tile<lmhead::Tile256x128>(a, s); break;
     case k256x160: launch_tile<lmhead::Tile256x160>(a, s); break;
     case k256x256: launch_tile<lmhead::Tile256x256>(a, s); break;
+    case kRowShapes: break;
   }
   return check_launch("row_gemm");
 }
@@ -1295,6 +1296,13 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
 extern "C" size_t sd_linear_workspace_size(int32_t rows, int32_t out_features, int32_t in_features) {
   if (rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % lmhead::kK) return 0;
   return linear_workspace(rows, in_features);
+}
+
+// Which kernel sd_linear runs for these sizes (RowShape). For this package's tests, which run each of them (not declared
+// in sd_attn.h).
+extern "C" int sd_linear_kernel(int32_t rows, int32_t out_features, int32_t in_features) {
+  if (rows <= 0 || out_features <= 0 || in_features <= 0 || in_features % lmhead::kK) return -1;
+  return row_plan(rows, out_features, in_features).shape;
 }
 
 extern "C" int sd_linear(const void* x, int64_t x_row_stride, int32_t rows, const void* packed_weight,

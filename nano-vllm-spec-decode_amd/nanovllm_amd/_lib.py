@@ -63,9 +63,10 @@ SIGNATURES = {
     "sd_sample": (_i32, [_c_void_p, _i32, _i64, _c_void_p, _c_void_p, _i32, _i32, _c_void_p, _c_void_p, _size,
                          _c_void_p]),
 }
-# Kernels of this package's own layers, not part of the C ABI.
+# For this package's own layers and tests, not part of the C ABI.
 INTERNAL = {
     "sd_silu_mul": (_i32, [_c_void_p, _i64, _i32, _i32, _c_void_p, _i64, _c_void_p]),
+    "sd_linear_kernel": (_i32, [_i32, _i32, _i32]),
 }
 
 _lib = None

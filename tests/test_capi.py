@@ -84,6 +84,17 @@ def test_lm_head_workspace_never_grew(lib):
     assert lib.sd_lm_head_verify_workspace_size(64, 4, 151936, 4096, 0) < 8 << 20
 
 
+def test_linear_edge_cases_reach_every_kernel(lib):
+    """The sizes that test_gpu_linear_norm.py compares at run each of sd_linear's 13 kernels: with more steps of 32
+    columns than the 16 that any keeps ahead, an odd number of them (a half stage) and so some left behind the main
+    loop; the one for ranges of a multiple of 16 steps with such ranges."""
+    from test_gpu_linear_norm import EDGE_ROWS, EDGES
+    seen = {lib.sd_linear_kernel(m, n, k) for n, k in EDGES for m in EDGE_ROWS if k // 32 > 16 and k // 32 % 2}
+    ranged = {lib.sd_linear_kernel(m, n, k) for n, k in EDGES for m in EDGE_ROWS if k // 32 % 128 == 0}
+    assert seen | {3} == set(range(13)) and 3 in ranged, (seen, ranged)
+    assert lib.sd_linear_kernel(0, 16, 32) == -1 == lib.sd_linear_kernel(1, 16, 33)
+
+
 def test_bad_arguments_return_status(lib):
     rc = lib.sd_store_kvcache(None, 0, None, 0, None, None, 0, None, -1, 8, 128, None)
     assert rc == 1 and b"bad sizes" in lib.sd_last_error()
