@@ -46,10 +46,19 @@ constexpr int kK = 32;                             // columns of a packed block:
 constexpr int kBlockBytes = kN * kK * 2;           // 16 KB: one step of a packed tile
 constexpr int kStreamRows = 16;                    // stream_gemm's token rows
 
-struct TileBest {  // first argmax of one token row over one workgroup's weight rows
+struct TileBest {  // first argmax of one token row over some weight rows; idx 0x7fffffff: nothing above -inf
   float val;
   int32_t idx;
 };
+// A workgroup's candidate in memory: the value, which is a bf16, and its index among the workgroup's weight rows
+// (0xffff: none). In four bytes, so that 128-row workgroups need no more of the caller's workspace than 256-row ones
+// with a whole TileBest.
+__device__ __forceinline__ uint32_t pack_best(float val, int32_t idx, int32_t first) {
+  return (__builtin_bit_cast(uint32_t, val) & 0xffff0000u) | (idx == 0x7fffffff ? 0xffffu : (uint32_t)(idx - first));
+}
+__device__ __forceinline__ TileBest unpack_best(uint32_t c, int32_t first) {
+  return {__builtin_bit_cast(float, c & 0xffff0000u), (c & 0xffff) == 0xffff ? 0x7fffffff : first + (int32_t)(c & 0xffff)};
+}
 
 struct Args {
   const uint16_t* x;        // [*, K] bf16 rows, stride x_stride
@@ -63,7 +72,7 @@ struct Args {
   int64_t out_stride;
   int32_t out_align;        // what out and its row stride are multiples of: 16, 8 or 2 bytes (8, 4 or 1 entries a store)
   int32_t out_nt;           // non-temporal stores of whole lines (logits: they leave the token rows in L2)
-  TileBest* best;           // [M][tiles_n], or null (no argmax)
+  uint32_t* best;           // [M][tiles_n] candidates (pack_best), or null (no argmax)
   int32_t tiles_n, tiles_m;
   int32_t full, splits;     // packed tiles from `full` on are summed in `splits` ranges of k, the others in one
 };
@@ -216,22 +225,50 @@ __device__ __forceinline__ bool row_valid(const Args& a, int m) {
   return r >= 0 && r < a.x_rows;
 }
 
-// Four consecutive entries n .. n + 3 of a token row, rounded to bf16 (zeros for an invalid row) and taken into the
-// running first argmax (index order within a lane: strictly larger).
-__device__ __forceinline__ uint2 round4(const Args& a, const f32x4& acc, bool valid, int n, float& bv, int& bi) {
-  uint2 w = make_uint2(cvt_bf16x2(acc[0], acc[1]), cvt_bf16x2(acc[2], acc[3]));
-  if (!valid) w = make_uint2(0, 0);
-  if (a.best) {
-    const float v[4] = {__builtin_bit_cast(float, w.x << 16), __builtin_bit_cast(float, w.x & 0xffff0000u),
-                        __builtin_bit_cast(float, w.y << 16), __builtin_bit_cast(float, w.y & 0xffff0000u)};
+// Four consecutive entries of a token row, rounded to bf16 (zeros for an invalid row).
+__device__ __forceinline__ uint2 round4(const f32x4& acc, bool valid) {
+  const uint2 w = make_uint2(cvt_bf16x2(acc[0], acc[1]), cvt_bf16x2(acc[2], acc[3]));
+  return valid ? w : make_uint2(0, 0);
+}
+// The first argmax (a NaN above all, nothing for -inf alone) of a lane's entries of one token row, w[i] those from
+// n + 16 i on. The maximum, then the first entry that equals it: about 3 instructions an entry. A running argmax takes
+// 9 in a chain, which one wave a SIMD cannot hide (3 us a workgroup of 256 x 160); it is left for waves with a NaN.
+template <int TN>
+__device__ __forceinline__ TileBest lane_best(const Args& a, const uint2 (&w)[TN], int n) {
+  float v[TN][4], top = -INFINITY;
+  bool nan = false;
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    v[i][0] = __builtin_bit_cast(float, w[i].x << 16);
+    v[i][1] = __builtin_bit_cast(float, w[i].x & 0xffff0000u);
+    v[i][2] = __builtin_bit_cast(float, w[i].y << 16);
+    v[i][3] = __builtin_bit_cast(float, w[i].y & 0xffff0000u);
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (n + e < a.N && bv == bv && !(v[e] <= bv)) {
-        bv = v[e];
-        bi = n + e;
-      }
+      if (n + 16 * i + e >= a.N) v[i][e] = -INFINITY;
+    nan |= __builtin_isunordered(v[i][0], v[i][1]) | __builtin_isunordered(v[i][2], v[i][3]);
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(top) : "v"(v[i][0]), "v"(v[i][1]));
+    asm("v_max3_f32 %0, %0, %1, %2" : "+v"(top) : "v"(v[i][2]), "v"(v[i][3]));
   }
-  return w;
+  TileBest b = {top, 0x7fffffff};
+  if (__builtin_amdgcn_ballot_w64(nan)) {
+    b.val = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool take = (b.val == b.val) & !(v[i][e] <= b.val);
+        b.val = take ? v[i][e] : b.val;
+        b.idx = take ? n + 16 * i + e : b.idx;
+      }
+    return b;
+  }
+#pragma unroll
+  for (int i = TN - 1; i >= 0; --i)
+#pragma unroll
+    for (int e = 3; e >= 0; --e) b.idx = v[i][e] == top ? n + 16 * i + e : b.idx;
+  b.idx = top == -INFINITY ? 0x7fffffff : b.idx;
+  return b;
 }
 // The first argmax over the four lanes that hold one token row's entries (l, l ^ 16, l ^ 32, l ^ 48).
 __device__ __forceinline__ void lanes_best(float& bv, int& bi) {
@@ -309,12 +346,11 @@ __global__ __launch_bounds__(kWave) void stream_gemm(Args a) {
       end_range(t + d);
     }
   const bool valid = row_valid(a, r16);
-  float bv = -INFINITY;
-  int bi = 0x7fffffff;
+  uint2 ws[TN];
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     const int n = n0 + 16 * i + 4 * g;
-    const uint2 w = round4(a, sum[i] + acc[i], valid, n, bv, bi);
+    const uint2 w = ws[i] = round4(sum[i] + acc[i], valid);
     if (!a.out || r16 >= a.M) continue;
     uint16_t* dst = a.out + (int64_t)r16 * a.out_stride + n;
     if (n + 3 < a.N && a.out_align >= 8) {
@@ -327,8 +363,9 @@ __global__ __launch_bounds__(kWave) void stream_gemm(Args a) {
     }
   }
   if (a.best) {
-    lanes_best(bv, bi);
-    if (g == 0 && r16 < a.M) a.best[(int64_t)r16 * a.tiles_n + blockIdx.x] = TileBest{bv, bi};
+    TileBest b = lane_best(a, ws, n0 + 4 * g);
+    lanes_best(b.val, b.idx);
+    if (g == 0 && r16 < a.M) a.best[(int64_t)r16 * a.tiles_n + blockIdx.x] = pack_best(b.val, b.idx, n0);
   }
 }
 
@@ -527,18 +564,18 @@ __global__ __launch_bounds__(T::kThreads, 1) void tile_gemm(Args a) {
   for (int j = 0; j < TM; ++j) {
     const int mr = wm * TM * 16 + 16 * j + r16;
     const bool valid = row_valid(a, m0 + mr);
-    float bv = -INFINITY;
-    int bi = 0x7fffffff;
+    uint2 ws[TN];
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const int nr = wn * TN * 16 + 16 * i + 4 * g;
       if constexpr (T::kSums) acc[i][j] = sum[i][j] + acc[i][j];   // the last range
-      const uint2 w = round4(a, acc[i][j], valid, nt * NT + nr, bv, bi);
-      *(uint2*)(lds + mr * (2 * NT) + (((nr / 8) ^ (mr & kSwz)) << 4) + 8 * (g % 2)) = w;
+      ws[i] = round4(acc[i][j], valid);
+      *(uint2*)(lds + mr * (2 * NT) + (((nr / 8) ^ (mr & kSwz)) << 4) + 8 * (g % 2)) = ws[i];
     }
     if (a.best) {
-      lanes_best(bv, bi);
-      if (g == 0) red[mr * WN + wn] = TileBest{bv, bi};
+      TileBest b = lane_best(a, ws, nt * NT + wn * TN * 16 + 4 * g);
+      lanes_best(b.val, b.idx);
+      if (g == 0) red[mr * WN + wn] = b;
     }
   }
   __syncthreads();
@@ -592,13 +629,15 @@ __global__ __launch_bounds__(T::kThreads, 1) void tile_gemm(Args a) {
       const TileBest o = red[mr * WN + w];
       if (better(o.val, o.idx, b.val, b.idx)) b = o;
     }
-    a.best[(int64_t)(m0 + mr) * a.tiles_n + nt] = b;
+    a.best[(int64_t)(m0 + mr) * a.tiles_n + nt] = pack_best(b.val, b.idx, nt * NT);
   }
 }
 
 // The workgroup shapes, smallest first: the larger, the less is loaded per MFMA (row_plan chooses). Tile32x64 has a
 // form for ranges that are multiples of its 16 register sets (Qwen3-8B's projections): with the check behind every
-// step 4096 x 12288 takes 42.0 us at 80 rows, with one in 16 steps 39.0, without ranges 38.2.
+// step 4096 x 12288 takes 42.0 us at 80 rows, with one in 16 steps 39.0, without ranges 38.2. Tile256x32 loads 3 steps
+// ahead, so that a CU holds three of its workgroups and 594 (the LM head) are one round: 151936 x 1024 at one row 54.9 us
+// with 7 steps ahead and two workgroups, 51.9 with 3; 151936 x 4096 194.1 and 191.7.
 typedef Tile<1, 4, 2, 1, 16, 9, false, false, true, 16> Tile32x64E16;
 typedef Tile<1, 4, 2, 1, 16, 9, false, false, true> Tile32x64;
 typedef Tile<1, 5, 2, 1, 16, 9, false, false, true> Tile32x80;
@@ -606,7 +645,7 @@ typedef Tile<1, 5, 4, 1, 8, 6, false, false, true> Tile64x80;
 typedef Tile<2, 4, 4, 1, 8, 6, false, false, true> Tile128x64;
 typedef Tile<2, 5, 4, 1, 8, 6, false, false, true> Tile128x80;
 typedef Tile<2, 10, 4, 1, 8, 6, false, true, false> Tile128x160;
-typedef Tile<4, 2, 4, 1, 8, 6, false, false, true> Tile256x32;
+typedef Tile<4, 2, 4, 1, 4, 6, false, false, true> Tile256x32;
 typedef Tile<4, 8, 4, 1, 4, 6, true, true, false> Tile256x128;
 typedef Tile<4, 10, 4, 1, 4, 6, true, true, true> Tile256x160;
 typedef Tile<4, 16, 4, 1, 4, 4, true, false, false, 0> Tile256x256;

@@ -905,14 +905,14 @@ int run_verify(const char* who, const void* logits, int32_t logits_dtype, int64_
 
 // The first argmax of each token row over the LM head's per-workgroup results, into the span statistics of
 // a one-span row (verify_decide reads them); one workgroup per row, any tree order (the argmax order is total).
-__global__ __launch_bounds__(kThreads) void lm_head_merge(const lmhead::TileBest* best, int tiles, RowStat* stats) {
+__global__ __launch_bounds__(kThreads) void lm_head_merge(const uint32_t* best, int tiles, int rows_n, RowStat* stats) {
   __shared__ float shv[4];
   __shared__ int shi[4];
   const int m = blockIdx.x;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
   for (int t = threadIdx.x; t < tiles; t += kThreads) {
-    const lmhead::TileBest b = best[(int64_t)m * tiles + t];
+    const lmhead::TileBest b = lmhead::unpack_best(best[(int64_t)m * tiles + t], t * rows_n);
     if (better(b.val, b.idx, bv, bi)) {
       bv = b.val;
       bi = b.idx;
@@ -944,35 +944,41 @@ enum RowShape { kStream16, kStream32, k256x32, k32x64E16, k32x64, k32x80, k64x80
                 k256x160, k256x256, kRowShapes };
 struct RowPlan {
   RowShape shape;
-  int tiles_n, tiles_m;
+  int rows_n, tiles_n, tiles_m;
 };
-// Up to 16 rows: stream_gemm, with 32 weight rows a wave from 192 waves on, but whole packed tiles from 512 tiles on
-// (the two workgroups a CU that fit then fill the GPU): 151936 x 4096 at 15 rows 207 us (199 without the logits)
-// against 216 (210) with stream_gemm, whose waves drift apart within a packed tile's block. More rows: the tile_gemm
-// shape with the least rounds of workgroups over the GPU x time of a workgroup, from each shape's measured time per
-// step of 32 columns (on all CUs, one workgroup each) and about 6 us of launch, first loads and epilogue, but never
-// less than the weight takes from HBM; of equal ones the first. A larger shape loads less per MFMA, a smaller one
-// keeps more CUs busy: at 320 rows 4096 x 4096 takes 25 us as 64 x 80 and 57 as 256 x 128, at 1168 rows
-// 24576 x 4096 207 us as 256 x 160 and 226 as 256 x 128. 256 x 256 has no registers for a sum of ranges: it takes
-// weights of one range a tile only (with its one-range sums 24576 x 4096 took 193 us). max_tiles: shapes that cut the
-// weight into more tiles are left out (it is at least the packed tiles, which the 256-row shapes have).
+// Up to 16 rows: stream_gemm, with 32 weight rows a wave from 192 waves on, but whole packed tiles from 192 tiles on,
+// which then fill the GPU: 151936 x 4096 at one row 192 us against 217 with stream_gemm, whose waves drift apart within
+// a packed tile's block, 49152 x 4096 58 against 67; below, 33024 x 3072 (129 tiles) 40 against 37.
+//
+// More rows: the tile_gemm shape of least time by this estimate, of equal ones the first. A call takes its rounds of
+// workgroups over the GPU (each XCD has the token tiles of an eighth of the weight tiles) times a shape's time per step
+// of 32 columns, at least the weight's time from HBM. What a workgroup needs besides (first loads, epilogue) is paid
+// every round by the shapes of which a CU holds one; where it holds more, one's start runs under another's steps. The
+// times are each shape's own, fitted to 1024, 4096 and 12288 columns. A larger shape loads less per MFMA, a smaller one keeps
+// more CUs busy: at 320 rows 4096 x 4096 takes 25 us as 64 x 80 and 57 as 256 x 128, at 1168 rows 24576 x 4096 207 us
+// as 256 x 160 and 226 as 256 x 128; 151936 x 1024 at 20 rows 54 as 128 x 64 and 77 as 256 x 128, whose three rounds
+// end with nothing to cover them; 151936 x 4096 at 160 rows 258 as 256 x 160 and 285 as 128 x 160. 256 x 256 has no
+// registers for a sum of ranges: it takes weights of one range a tile only (with its one-range sums 24576 x 4096 took
+// 193 us). max_tiles: shapes that cut the weight into more tiles are left out (it is at least the packed tiles, which
+// the 256-row shapes have).
 RowPlan row_plan(int M, int N, int K, int max_tiles = INT32_MAX) {
   if (M <= lmhead::kStreamRows) {
-    const bool wide = N >= 192 * 32;
-    const int stream_tiles = (N + (wide ? 31 : 15)) / (wide ? 32 : 16);
-    if (N >= 512 * lmhead::kN || stream_tiles > max_tiles) return {k256x32, (N + lmhead::kN - 1) / lmhead::kN, 1};
-    return {wide ? kStream32 : kStream16, stream_tiles, 1};
+    const int rows_n = N >= 192 * 32 ? 32 : 16, tiles = (N + rows_n - 1) / rows_n;
+    if (N >= 192 * lmhead::kN || tiles > max_tiles) return {k256x32, lmhead::kN, (N + lmhead::kN - 1) / lmhead::kN, 1};
+    return {rows_n == 32 ? kStream32 : kStream16, rows_n, tiles, 1};
   }
   struct Shape {
     RowShape shape;
-    int rows_n, rows_m, step_ns, ends;   // ranges end at multiples of `ends` steps (0: one range only)
+    int rows_n, rows_m, step_ns, start_ns;
+    int per_cu;   // workgroups of a CU whose starts overlap
+    int ends;     // ranges end at multiples of `ends` steps (0: one range only)
   };
   static constexpr Shape kShapes[] = {
-      {k32x64E16, 32, 64, 100, 16}, {k32x64, 32, 64, 100, 1},     {k32x80, 32, 80, 125, 1},
-      {k64x80, 64, 80, 156, 1},     {k128x64, 128, 64, 210, 1},   {k128x80, 128, 80, 235, 1},
-      {k128x160, 128, 160, 290, 1}, {k256x128, 256, 128, 420, 1}, {k256x160, 256, 160, 560, 1},
-      {k256x256, 256, 256, 760, 0}};
-  constexpr int kCUs = 256, kStartNs = 6000, kHbmBytesPerNs = 5600;
+      {k32x64E16, 32, 64, 100, 5000, 2, 16},  {k32x64, 32, 64, 105, 5000, 2, 1},    {k32x80, 32, 80, 117, 6500, 1, 1},
+      {k64x80, 64, 80, 165, 5000, 2, 1},      {k128x64, 128, 64, 260, 3000, 3, 1},  {k128x80, 128, 80, 265, 6000, 2, 1},
+      {k256x32, 256, 32, 320, 3500, 2, 1},    {k128x160, 128, 160, 318, 7000, 1, 1}, {k256x128, 256, 128, 470, 8000, 1, 1},
+      {k256x160, 256, 160, 540, 9000, 1, 1},  {k256x256, 256, 256, 660, 10000, 1, 0}};
+  constexpr int kXcds = 8, kXcdCUs = 32, kHbmBytesPerNs = 6200;
   const int64_t hbm_ns = (int64_t)N * K * 2 / kHbmBytesPerNs;
   const int splits = lmhead::sum_ranges(N, K).splits, steps = K / lmhead::kK;
   RowPlan best{};
@@ -982,11 +988,12 @@ RowPlan row_plan(int M, int N, int K, int max_tiles = INT32_MAX) {
     if (splits > 1 && (c.ends == 0 || (c.ends > 1 && steps % (splits * c.ends)))) continue;
     const int tn = (N + c.rows_n - 1) / c.rows_n, tm = (M + c.rows_m - 1) / c.rows_m;
     if (tn > max_tiles) continue;
-    const int64_t rounds = ((int64_t)tn * tm + kCUs - 1) / kCUs;
-    const int64_t ns = std::max(hbm_ns, rounds * ((int64_t)steps * c.step_ns + kStartNs));
+    const int64_t rounds = ((int64_t)((tn + kXcds - 1) / kXcds) * tm + kXcdCUs - 1) / kXcdCUs;
+    const int64_t ns =
+        std::max(hbm_ns, rounds * steps * c.step_ns) + (rounds + c.per_cu - 1) / c.per_cu * c.start_ns;
     if (ns < best_ns) {
       best_ns = ns;
-      best = {c.shape, tn, tm};
+      best = {c.shape, c.rows_n, tn, tm};
     }
   }
   return best;
@@ -1068,15 +1075,15 @@ LmLayout lm_layout(int S, int K, int V, int H) {
   LmLayout L;
   L.overlap_tiles = (V + lmhead::kN - 1) / lmhead::kN;
   // Never more than a caller may have been told for these sizes when the workspace held the candidates of 256-row tiles
-  // and the rows, packed and padded to 64: shapes of more tiles are left out where they would take more (calls of few
-  // hidden columns or a very wide vocabulary).
+  // (8 bytes) and the rows, packed and padded to 64: shapes of more tiles are left out where they would take more (calls
+  // of few hidden columns or a very wide vocabulary).
   const int64_t packed = (M + 63) / 64 * 64 * H * 2;
-  L.max_tiles = (int)std::min<int64_t>(L.overlap_tiles + packed / (M * (int64_t)sizeof(lmhead::TileBest)), INT32_MAX);
+  L.max_tiles = (int)std::min<int64_t>(2 * (int64_t)L.overlap_tiles + packed / (M * (int64_t)sizeof(uint32_t)), INT32_MAX);
   L.stats = 0;
   L.info = align256((size_t)M * sizeof(RowStat));
   L.best = align256(L.info + (size_t)S * sizeof(SeqInfo));
-  L.copy = align256(L.best + (size_t)M * L.overlap_tiles * sizeof(lmhead::TileBest));
-  const size_t best = (size_t)M * row_plan(rows, V, H, L.max_tiles).tiles_n * sizeof(lmhead::TileBest);
+  L.copy = align256(L.best + (size_t)M * L.overlap_tiles * sizeof(uint32_t));
+  const size_t best = (size_t)M * row_plan(rows, V, H, L.max_tiles).tiles_n * sizeof(uint32_t);
   L.total = std::max(align256(L.best + best), align256(L.copy + (size_t)M * H * 2));
   return L;
 }
@@ -1253,7 +1260,7 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
   a.out_stride = logits_out_row_stride;
   a.out_align = row_align(logits_out, logits_out_row_stride);
   a.out_nt = 1;  // 64 rows with their logits 237.7 -> 221.6 us, 80 rows 244.7 -> 229.0
-  a.best = temperatures ? nullptr : (lmhead::TileBest*)((uint8_t*)workspace + lay.best);
+  a.best = temperatures ? nullptr : (uint32_t*)((uint8_t*)workspace + lay.best);
   const bool overlap =
       logits_out && rows_overlap(hidden, hidden_rows, hidden_row_stride, H, logits_out, M, logits_out_row_stride, V);
   const RowPlan plan = row_plan(a.M, V, H, !a.best ? INT32_MAX : overlap ? lay.overlap_tiles : lay.max_tiles);
@@ -1286,7 +1293,8 @@ extern "C" int sd_lm_head_verify(const void* hidden, int64_t hidden_row_stride, 
   p.out_next = next_token;
   p.stats = (RowStat*)((uint8_t*)workspace + lay.stats);
   p.info = (SeqInfo*)((uint8_t*)workspace + lay.info);
-  hipLaunchKernelGGL(lm_head_merge, dim3((unsigned)M), dim3(kThreads), 0, s, a.best, plan.tiles_n, p.stats);
+  hipLaunchKernelGGL(lm_head_merge, dim3((unsigned)M), dim3(kThreads), 0, s, a.best, plan.tiles_n, plan.rows_n,
+                     p.stats);
   if ((rc = check_launch("lm_head_merge"))) return rc;
   hipLaunchKernelGGL((verify_decide<SD_DTYPE_BF16, SD_DTYPE_BF16, false>), dim3(S), dim3(64), 0, s, p);
   if ((rc = check_launch("verify_decide"))) return rc;

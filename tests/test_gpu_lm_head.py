@@ -242,3 +242,34 @@ def test_lm_head_workspace_and_logits_over_hidden(device, monkeypatch, S, K, V, 
     assert bool((buf[asked[0]:] == 0x5a).all())
     ref_acc, ref_nxt = osmp.verify_drafts(want.cpu(), drafts.cpu(), nd.cpu(), zeros.cpu())
     assert torch.equal(acc.cpu(), ref_acc) and torch.equal(nxt.cpu(), ref_nxt)
+
+
+@pytest.mark.parametrize("V", [1003, 9001, 40005, 131075])
+def test_lm_head_argmax_of_special_values(device, V):
+    """The epilogue's argmax is torch.argmax's (the first of equal entries, a NaN above all) on rows of zeros, ties,
+    infinities, NaN before and after infinities, zeros of both signs and a maximum at the ragged end, in every kernel's
+    place for 1 to 400 rows. Infinities and NaN come from overflowing products: weights and rows are finite."""
+    H, big = 64, 3e38
+    g = torch.Generator().manual_seed(V)
+    w = torch.zeros(V, H)
+    x = torch.zeros(9, H)                        # row 0: all zeros
+    w[:, 1], x[1, 1] = torch.randint(0, 3, (V,), generator=g).float(), 1.0
+    w[V // 2, 2], w[V // 2 + 70, 2], x[2, 2] = big, big, big                    # two infinities
+    w[V // 3, 3], w[V // 3, 4], w[V // 3 + 5, 3], w[7, 3] = big, -big, big, big  # NaN between infinities
+    x[3, 3] = x[3, 4] = big
+    w[V - 3, 5], w[V - 3, 6], w[V - 2, 5], w[V - 2, 6], x[4, 5:7] = big, -big, big, -big, big   # two NaN at the end
+    w[:, 7], x[5, 7] = torch.where(torch.rand(V, generator=g) < 0.5, 0.0, -1.0), -1.0         # zeros of both signs, ones
+    w[:, 8], x[6, 8] = -1.0 - torch.rand(V, generator=g), 1.0                   # all negative
+    w[:, 9], w[V - 1, 9], x[7, 9] = torch.rand(V, generator=g), 2.0, 1.0        # the last entry
+    w[:, 10], w[V // 2, 10], x[8, 10] = big, 0.0, -big                          # -inf everywhere but at one entry
+    head = LMHeadVerifier(w.to(torch.bfloat16).to(device))
+    for M in (1, 9, 16, 17, 40, 80, 160, 400):
+        pick = torch.arange(M) % 9 if M > 1 else torch.tensor([3])
+        h = x[pick].to(torch.bfloat16).to(device)
+        out = torch.empty(M, V, dtype=torch.bfloat16, device=device)
+        nxt = lm_head_sample(h, head, torch.zeros(M, device=device), logits_out=out)
+        logits = out.float().cpu()
+        want = logits.argmax(-1)
+        assert torch.equal(nxt.cpu(), want), (M, nxt.cpu()[:9], want[:9])
+        if M >= 9:
+            assert logits[2].isinf().any() and logits[3].isnan().sum() == 1 and logits[4].isnan().sum() == 2
