@@ -1505,7 +1505,8 @@ int residue_waves(int64_t items, int Hkv, int RT) {
 // 10.8, 3 x 2000 the same, 8 x 300 9.1 -> 9.5; more than a pass: 20 rows, 1 x 4096 19.5 -> 20.5, 4 x 2000
 // 18.9 -> 21.8; 36 rows, 2 x 1000 11.5 -> 14.8. The line is in pairs, which is what fills the GPU, but only 8, 16,
 // 24, 64 and 128 pairs were measured, all of 8 KV heads: not other head counts with as many pairs (two sequences of 4 KV
-// heads are 8 too) nor the counts between; in 16 to 64 pairs neither form was ahead by more than 8 %. (Calls of at least kArrivals pairs have eight waves, or four row tiles.)
+// heads are 8 too) nor the counts between; in 16 to 64 pairs neither form was ahead by more than 8 %.
+// (Calls of at least kArrivals pairs have eight waves, or four row tiles.)
 bool merges_last(int waves, int64_t pairs, int merge_rows) {
   const int threads = waves == 1 ? kStreamThreads : waves * kWave;
   return pairs <= kArrivals && (waves == 4 || (waves == 1 && pairs <= 8)) && merge_rows * (kD / 4) <= threads;

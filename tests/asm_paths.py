@@ -90,16 +90,10 @@ def _all_regs(text):
     return out
 
 
-def unsafe_in_flight(ins):
-    """Inline-asm loads (global_load_dwordx4 counted by vmcnt, ds_read_b128 by lgkmcnt) whose destination an
-    instruction names before a wait covers the load, over every path of the control flow graph: at each point the
-    fewest instructions of the load's counter issued after it on any path to that point. A wait for N covers a load
-    with at least N such instructions after it. Only LDS instructions count for lgkmcnt (scalar loads return out of
-    order). Returns ([(load, index, touching instruction)], global loads, LDS reads)."""
-    cap = 64
+def _successors(ins):
     labels = {t.split(":")[0]: i for i, (t, _) in enumerate(ins) if re.match(r"\.L\w+:", t)}
-    ops, succ = [], []
-    for i, (t, in_asm) in enumerate(ins):
+    succ = []
+    for i, (t, _) in enumerate(ins):
         nxt = [i + 1] if i + 1 < len(ins) else []
         m = re.match(r"s_(cbranch_\w+|branch)\s+(\.L\S+)", t)
         if m:
@@ -107,6 +101,51 @@ def unsafe_in_flight(ins):
         else:
             assert not re.match(r"s_(setpc|swappc|call)", t), t
             succ.append([] if t.startswith("s_endpgm") else nxt)
+    return succ
+
+
+def early_mfma_reads(ins, states=18):
+    """[(mfma, index, touching instruction)]: results of inline-asm MFMAs, whose latency the compiler does not know,
+    named by another instruction than an MFMA fewer than `states` wait states after it on some path (an instruction
+    counts one, s_nop N one more than N; a 16-pass MFMA's result needs 18 before the VALU or memory reads it)."""
+    succ, state, work, bad = _successors(ins), {0: {}}, [0], {}
+    while work:
+        i = work.pop()
+        t, in_asm = ins[i]
+        name, _, args = t.partition(" ")
+        mfma = name.startswith("v_mfma")
+        if not (mfma or name.startswith("s_") or re.match(r"\.L\w+:", t)):
+            for r in _all_regs(args) & state[i].keys():
+                bad.setdefault((state[i][r][1], i), (ins[state[i][r][1]][0], state[i][r][1], t))
+        step = int(args) + 1 if name == "s_nop" else 0 if re.match(r"\.L\w+:", t) else 1
+        cur = {r: (n + step, j) for r, (n, j) in state[i].items() if n + step < states}
+        if mfma and in_asm:
+            cur.update({r: (0, i) for r in _all_regs(args.split(",")[0])})
+        for j in succ[i]:
+            old = state.setdefault(j, None)
+            if old is None:
+                state[j] = dict(cur)
+                work.append(j)
+                continue
+            changed = False
+            for r, v in cur.items():
+                if r not in old or v[0] < old[r][0]:
+                    old[r] = v
+                    changed = True
+            if changed:
+                work.append(j)
+    return sorted(bad.values(), key=lambda x: x[1])
+
+
+def unsafe_in_flight(ins):
+    """Inline-asm loads (global_load_dwordx4 counted by vmcnt, ds_read_b128 by lgkmcnt) whose destination an
+    instruction names before a wait covers the load, over every path of the control flow graph: at each point the
+    fewest instructions of the load's counter issued after it on any path to that point. A wait for N covers a load
+    with at least N such instructions after it. Only LDS instructions count for lgkmcnt (scalar loads return out of
+    order). Returns ([(load, index, touching instruction)], global loads, LDS reads)."""
+    cap = 64
+    ops, succ = [], _successors(ins)
+    for t, in_asm in ins:
         name, _, args = t.partition(" ")
         if re.match(r"\.L\w+:", t):
             ops.append(("none",))

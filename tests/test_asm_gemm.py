@@ -1,7 +1,8 @@
 """tile_gemm issues its weight loads and LDS reads as inline asm, which the compiler does not know to be in flight.
 Compiles verify_sampler.hip (hipcc, no GPU) and checks every instantiation's gfx950 code: no destination register
 of a weight load (global_load_dwordx4) or an LDS read (ds_read_b128) is read, copied or reused on any path before a
-wait that covers the load, and nothing is spilled (a spill could store a register whose load has not landed)."""
+wait that covers the load, no MFMA's result is read before it is there, and nothing is spilled (a spill could store
+a register whose load has not landed)."""
 import os
 import re
 import shutil
@@ -15,7 +16,7 @@ PKG = os.path.join(ROOT, "nano-vllm-spec-decode_amd")
 sys.path.insert(0, PKG)
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 
-from asm_paths import function_lines, unsafe_in_flight  # noqa: E402
+from asm_paths import early_mfma_reads, function_lines, unsafe_in_flight  # noqa: E402
 
 
 @pytest.fixture(scope="module")
@@ -47,6 +48,19 @@ def test_tile_gemm_loads_complete_before_use(device_asm):
         assert not bad, (symbol, bad[:4])
         scratch = re.search(r"; ScratchSize: (\d+)", device_asm[device_asm.index("\n" + symbol + ":"):])
         assert scratch and int(scratch.group(1)) == 0, symbol
+
+
+def test_tile_gemm_waits_for_its_mfmas(device_asm):
+    """The MFMAs are inline asm too: nothing but an MFMA touches a result before it is there (the sums between two
+    ranges and the epilogue wait by s_nop), in every instantiation. Without those waits the check finds reads too early
+    in the shape that has the fewest instructions between."""
+    found = 0
+    for symbol in _kernels(device_asm):
+        lines = function_lines(device_asm, symbol)
+        bad = early_mfma_reads(lines)
+        assert not bad, (symbol, bad[:4])
+        found += len(early_mfma_reads([(t, a) for t, a in lines if t != "s_nop 15"]))
+    assert found
 
 
 def test_check_finds_a_wait_too_short(device_asm):
